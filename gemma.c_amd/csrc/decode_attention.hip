@@ -24,8 +24,7 @@
 // stored split maxima are converted back to the reference's natural-log units.
 #include "gemma4_device.hpp"
 #include "decode_common.hpp"
-#include "lds_copy.hpp"
-#include "prep_common.hpp"
+#include "decode_row.hpp"
 
 #include "gemma4_flash_attention.h"
 
@@ -90,9 +89,6 @@ struct DecodeShape {
   // global one (src/gemma4.h rotary settings).
   static constexpr int kRot = kHeads == 1 ? kDim / 4 : kDim;
   static constexpr int kMaxW = kWaves;  // waves of a split workgroup at most
-  // Staged shapes: two waves per head group take alternate 8-key tiles that
-  // the workgroup copies into LDS once (all heads read every key).
-  static constexpr bool kStaged = kWaves == 2 * HG;
   static_assert(G % GW == 0, "heads per wave must divide the GQA group");
   static_assert(NP <= LPR, "one reduced score per lane at most");
   static_assert((NP & (NP - 1)) == 0 && (GW & (GW - 1)) == 0, "powers of two");
@@ -100,194 +96,6 @@ struct DecodeShape {
   static_assert(RPL * NP <= kWave, "probability slot holds one tile");
 };
 
-
-// Log-sum-exp combine of `splits` partials for GW consecutive query heads
-// starting at q_head0 of batch b, by one wave of the last-arriving split
-// workgroup, reading the other workgroups' partials with coherent loads that
-// are issued in independent batches (one memory round trip per batch).
-// Lane (r, cpack) owns dims [8*cpack, 8*cpack+8) and takes the splits
-// s == r (mod RPL); the RPL row groups are summed at the end. Same
-// arithmetic as decode_combine_kernel.
-template <int GW, int D, int LPR, int RPL>
-__device__ __forceinline__ void combine_row_group(const DecodeParams &p, int32_t b,
-                                                  int32_t q_head0, int32_t splits,
-                                                  int r, int cpack) {
-  constexpr int kBatch = 8;
-  const int lane = __lane_id();
-#pragma unroll 1
-  for (int g = 0; g < GW; ++g) {
-    const int64_t row = (int64_t)b * kQueryHeads + q_head0 + g;
-    const auto pm = coherent_view(p.partial_m + row * p.num_splits, splits);
-    const auto pl = coherent_view(p.partial_l + row * p.num_splits, splits);
-    const auto pa = coherent_view(p.partial_acc + row * p.num_splits * D, splits * D);
-    float big_m = -INFINITY;
-    for (int32_t s0 = 0; s0 < splits; s0 += kWave * 4) {
-      float mv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int32_t s = s0 + i * kWave + lane;
-        mv[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(pm, s * 4, 0, kCoherentAux));
-        mv[i] = s < splits ? mv[i] : -INFINITY;
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) big_m = fmaxf(big_m, mv[i]);
-    }
-    big_m = reduce_max_from<1>(big_m);
-    float big_l = 0.0f;
-    float sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int32_t s0 = r; s0 < splits; s0 += kBatch * RPL) {
-      float ms[kBatch], ls[kBatch];
-      u32x4 lo[kBatch], hi[kBatch];
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        const int32_t s = s0 + i * RPL;  // past `splits`: reads 0, weight 0
-        ms[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(pm, s * 4, 0, kCoherentAux));
-        ls[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(pl, s * 4, 0, kCoherentAux));
-        const int32_t off = (s * D + cpack * 8) * 4;
-        lo[i] = __builtin_amdgcn_raw_buffer_load_b128(pa, off, 0, kCoherentAux);
-        hi[i] = __builtin_amdgcn_raw_buffer_load_b128(pa, off + 16, 0, kCoherentAux);
-      }
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        const float w = ls[i] > 0.0f ? __builtin_amdgcn_exp2f((ms[i] - big_m) * kLog2e) : 0.0f;
-        big_l = fmaf(ls[i] > 0.0f ? ls[i] : 0.0f, w, big_l);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          sum[j] = fmaf(__uint_as_float(lo[i][j]), w, sum[j]);
-          sum[4 + j] = fmaf(__uint_as_float(hi[i][j]), w, sum[4 + j]);
-        }
-      }
-    }
-    big_l = sum_rows<LPR>(big_l);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sum[j] = sum_rows<LPR>(sum[j]);
-    if (r == 0) {
-      const float inv = (splits > 0 && big_l > 0.0f) ? 1.0f / big_l : 0.0f;
-      uint4 o;
-      o.x = pack_bf16x2(sum[0] * inv, sum[1] * inv);
-      o.y = pack_bf16x2(sum[2] * inv, sum[3] * inv);
-      o.z = pack_bf16x2(sum[4] * inv, sum[5] * inv);
-      o.w = pack_bf16x2(sum[6] * inv, sum[7] * inv);
-      store128(p.out + row * D + cpack * kPackElems, o);
-    }
-  }
-}
-
-// RMSNorm (learned weight, or scale-free with weight == null) and split-half
-// RoPE over the first kRot dims of one head held in this kernel's layout:
-// lane c of a row holds dims [8c, 8c + 8) of the D = 8 * LPR dims, so the sum
-// of squares is a reduction over the LPR lanes of the row and the rotary
-// partner of dim d (d + kRot/2 or d - kRot/2) sits kRot/16 lanes away.
-// Follows src/gemma4_flash_attention_decode.cu:233-283 and
-// src/gemma4_rope.cu:8-20; the result is rounded to bf16 as the reference
-// stores prepared rows.
-template <int LPR, int kRot>
-__device__ __forceinline__ uint4 prep_pack(uint4 raw, const uint16_t *weight,
-                                           const float *cos_row, const float *sin_row,
-                                           int cpack) {
-  float x[8];
-  unpack8(raw, x);
-  float ss = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ss = fmaf(x[i], x[i], ss);
-  ss += lane_xor<1>(ss);
-  ss += lane_xor<2>(ss);
-  ss += lane_xor<4>(ss);
-  ss += lane_xor<8>(ss);
-  ss = xor_sum<16>(ss);
-  if constexpr (LPR == 64) ss = xor_sum<32>(ss);
-  const float scale = 1.0f / sqrtf(ss / (float)(LPR * kPackElems) + kRmsEps);
-  float y[8];
-  if (weight == nullptr) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = x[i] * scale;
-  } else {
-    float w[8];
-    unpack8(load128(weight + cpack * kPackElems), w);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = x[i] * scale * w[i];
-    constexpr int kHalf = kRot / 2;
-    float partner[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) partner[i] = lane_xor<kHalf / kPackElems>(y[i]);
-    const int d0 = cpack * kPackElems;
-    if (d0 < kRot) {
-      const int pair = d0 < kHalf ? d0 : d0 - kHalf;
-      const float sign = d0 < kHalf ? -1.0f : 1.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) y[i] = fmaf(sign * partner[i], sin_row[pair + i], y[i] * cos_row[pair + i]);
-    }
-  }
-  return make_uint4(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]), pack_bf16x2(y[4], y[5]),
-                    pack_bf16x2(y[6], y[7]));
-}
-
-// The inputs prep_pack reads besides the row, loaded ahead of the math: the
-// lane's 8 weights (packed bf16) and cos / sin of its rotary pair.
-struct PrepInputs {
-  uint4 w;
-  float4 c0, c1, s0, s1;
-};
-template <int LPR, int kRot>
-__device__ __forceinline__ PrepInputs prep_inputs(const uint16_t *weight, const float *cos_row,
-                                                  const float *sin_row, int cpack) {
-  PrepInputs in;
-  in.w = weight != nullptr ? load128(weight + cpack * kPackElems) : make_uint4(0, 0, 0, 0);
-  const int d0 = cpack * kPackElems;
-  const int pair = d0 < kRot / 2 ? d0 : d0 - kRot / 2;
-  const bool rot = weight != nullptr && d0 < kRot;
-  // Scalar loads: the tables come through the C-ABI with no alignment promise.
-  const float *cr = rot ? cos_row + pair : nullptr;
-  const float *sr = rot ? sin_row + pair : nullptr;
-  in.c0 = rot ? make_float4(cr[0], cr[1], cr[2], cr[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
-  in.c1 = rot ? make_float4(cr[4], cr[5], cr[6], cr[7]) : make_float4(0.f, 0.f, 0.f, 0.f);
-  in.s0 = rot ? make_float4(sr[0], sr[1], sr[2], sr[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
-  in.s1 = rot ? make_float4(sr[4], sr[5], sr[6], sr[7]) : make_float4(0.f, 0.f, 0.f, 0.f);
-  return in;
-}
-// prep_pack's arithmetic on preloaded inputs (weighted: learned RMSNorm +
-// RoPE; otherwise the scale-free RMSNorm), the same operations in the same
-// order.
-template <int LPR, int kRot>
-__device__ __forceinline__ uint4 prep_math(uint4 raw, bool weighted, const PrepInputs &in,
-                                           int cpack) {
-  float x[8];
-  unpack8(raw, x);
-  float ss = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ss = fmaf(x[i], x[i], ss);
-  ss += lane_xor<1>(ss);
-  ss += lane_xor<2>(ss);
-  ss += lane_xor<4>(ss);
-  ss += lane_xor<8>(ss);
-  ss = xor_sum<16>(ss);
-  if constexpr (LPR == 64) ss = xor_sum<32>(ss);
-  const float scale = 1.0f / sqrtf(ss / (float)(LPR * kPackElems) + kRmsEps);
-  float y[8];
-  if (!weighted) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = x[i] * scale;
-  } else {
-    float w[8];
-    unpack8(in.w, w);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = x[i] * scale * w[i];
-    constexpr int kHalf = kRot / 2;
-    float partner[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) partner[i] = lane_xor<kHalf / kPackElems>(y[i]);
-    const int d0 = cpack * kPackElems;
-    if (d0 < kRot) {
-      const float sign = d0 < kHalf ? -1.0f : 1.0f;
-      const float c[8] = {in.c0.x, in.c0.y, in.c0.z, in.c0.w, in.c1.x, in.c1.y, in.c1.z, in.c1.w};
-      const float sn[8] = {in.s0.x, in.s0.y, in.s0.z, in.s0.w, in.s1.x, in.s1.y, in.s1.z, in.s1.w};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) y[i] = fmaf(sign * partner[i], sn[i], y[i] * c[i]);
-    }
-  }
-  return make_uint4(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]), pack_bf16x2(y[4], y[5]),
-                    pack_bf16x2(y[6], y[7]));
-}
 
 template <class Sh>
 __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeParams p) {
@@ -298,19 +106,7 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
   __shared__ int32_t s_rows[Sh::kMaxW][2][kWave];
   __shared__ float s_prob[Sh::kMaxW][kWave];
   __shared__ float s_ml[Sh::kMaxW][2][GW];
-  // Staged shapes: kStages stages of K and V rows for kStepKeys keys (one
-  // KT-key tile per key lane per step), rows of kWindowKeys keys at a time.
-  constexpr int kStages = 2;
-  constexpr int kLanes = Sh::kMaxW / HG;  // key lanes: tiles per step
-  constexpr int kStepKeys = kLanes * KT;
-  constexpr int kWindowKeys = Sh::kMaxW * kWave;
-  constexpr int kStageUint4 = Sh::kStaged ? kStages * 2 * kStepKeys * LPR : 0;
-  constexpr int kAccUint4 = Sh::kMaxW * GW * D / 4;
-  // The cross-wave merge buffer s_acc shares LDS with the stages: the merge
-  // runs after the last step's barrier.
-  __shared__ __attribute__((aligned(1024)))
-  uint4 s_lds[kStageUint4 > kAccUint4 ? kStageUint4 : kAccUint4];
-  auto s_acc = reinterpret_cast<float (*)[GW][D]>(&s_lds[0]);
+  __shared__ __attribute__((aligned(16))) float s_acc[Sh::kMaxW][GW][D];  // cross-wave merge
 
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = wave_uniform(threadIdx.x / kWave);  // scalar: wave-uniform control flow
@@ -348,9 +144,9 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
   const int32_t seq_word = p.seq_lengths[b];
   const int32_t tok_word = *tok_src;
   const int32_t gate_word = *gate_src;
-  const int32_t early_page = Sh::kStaged ? 0
-      : p.page_table[b * c.max_pages_per_seq +
-                     (int32_t)((key0 / c.page_size) % c.max_pages_per_seq)];
+  const int32_t early_page =
+      p.page_table[b * c.max_pages_per_seq +
+                   (int32_t)((key0 / c.page_size) % c.max_pages_per_seq)];
   const int32_t seq_len = wave_uniform(seq_word);
   const int32_t token_pos = p.token_position != nullptr ? wave_uniform(tok_word) : -1;
   int32_t first = c.window_size > 0 ? seq_len - c.window_size : 0;
@@ -358,9 +154,8 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
   const int32_t key_count = seq_len > first ? seq_len - first : 0;
   const int32_t live_splits = (key_count + p.split_size - 1) / p.split_size;
   const bool direct = p.num_splits == 1;
-  const bool by_slot =
-      !Sh::kStaged && p.slot_splits != 0 && c.window_size > 0 && key_count == ring_keys;
-  const bool early_ok = !Sh::kStaged && (c.window_size == 0 || by_slot);
+  const bool by_slot = p.slot_splits != 0 && c.window_size > 0 && key_count == ring_keys;
+  const bool early_ok = c.window_size == 0 || by_slot;
 
   if (p.gate != nullptr && wave_uniform(gate_word) != 0) {
     // A failed step: no append; a direct launch zeroes its rows (the
@@ -503,10 +298,6 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
       qw[g][0] = qp.x; qw[g][1] = qp.y; qw[g][2] = qp.z; qw[g][3] = qp.w;
     }
   };
-  auto load_q = [&]() __attribute__((always_inline)) {
-    q_issue();
-    q_finish();
-  };
 
   // Score-lane identity after the butterfly: one (key, head) per lane.
   const int idx = cpack >> S;               // index into the lane's NP partials
@@ -645,134 +436,22 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[g][j] *= alpha[g];
     }
-    if constexpr (GW >= 4) {
-      // GQA-heavy shapes (the 1x512 geometry's 16 heads per KV head are
-      // VALU-bound): P.V on v_dot2 over key pairs (kl, kl + 1), with bf16
-      // probability pairs and the V words regrouped by dim with one byte
-      // permute per word pair (28.8 against 31.6 us at 8193 keys). The 8x256
-      // shape keeps the fp32 FMA form: the dot2 form measured 1.7% slower on
-      // the HBM-bound batch-64 leg.
-      // Staged tiles hold zero rows for unreadable keys (their probability
-      // is 0 as well), so only register-loaded tiles mask V.
 #pragma unroll
-      for (int kl = 0; kl < LOADS; kl += 2) {
-        const bool ok0 = Sh::kStaged || ((t.valid >> kl) & 1u);
-        const bool ok1 = Sh::kStaged || ((t.valid >> (kl + 1)) & 1u);
-        const uint32_t a[4] = {ok0 ? t.v[kl].x : 0u, ok0 ? t.v[kl].y : 0u, ok0 ? t.v[kl].z : 0u,
-                               ok0 ? t.v[kl].w : 0u};
-        const uint32_t c[4] = {ok1 ? t.v[kl + 1].x : 0u, ok1 ? t.v[kl + 1].y : 0u,
-                               ok1 ? t.v[kl + 1].z : 0u, ok1 ? t.v[kl + 1].w : 0u};
-        uint32_t pp[GW];
+    for (int kl = 0; kl < LOADS; ++kl) {
+      float vf[8];
+      const bool kl_valid = (t.valid >> kl) & 1u;
+      const uint4 vp = kl_valid ? t.v[kl] : make_uint4(0, 0, 0, 0);
+      unpack8(vp, vf);
 #pragma unroll
-        for (int g = 0; g < GW; ++g) {
-          const bf16x2_t pair = {(__bf16)pv[kl * GW + g], (__bf16)pv[(kl + 1) * GW + g]};
-          pp[g] = __builtin_bit_cast(uint32_t, pair);
-        }
+      for (int g = 0; g < GW; ++g) {
+        const float w = pv[kl * GW + g];
 #pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-          const uint32_t lo = __builtin_amdgcn_perm(c[wi], a[wi], 0x05040100u);
-          const uint32_t hi = __builtin_amdgcn_perm(c[wi], a[wi], 0x07060302u);
-#pragma unroll
-          for (int g = 0; g < GW; ++g) {
-            acc[g][2 * wi] = dot2_bf16(pp[g], lo, acc[g][2 * wi]);
-            acc[g][2 * wi + 1] = dot2_bf16(pp[g], hi, acc[g][2 * wi + 1]);
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int kl = 0; kl < LOADS; ++kl) {
-        float vf[8];
-        const bool kl_valid = (t.valid >> kl) & 1u;
-        const uint4 vp = kl_valid ? t.v[kl] : make_uint4(0, 0, 0, 0);
-        unpack8(vp, vf);
-#pragma unroll
-        for (int g = 0; g < GW; ++g) {
-          const float w = pv[kl * GW + g];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc[g][j] = fmaf(w, vf[j], acc[g][j]);
-        }
+        for (int j = 0; j < 8; ++j) acc[g][j] = fmaf(w, vf[j], acc[g][j]);
       }
     }
   };
 
-  if constexpr (Sh::kStaged) {
-    // Every head group (the 1 x 512 geometry: four groups of four heads)
-    // attends to every key of the split, so each step of kStepKeys keys (one
-    // KT-key tile per key lane) is copied into LDS once per workgroup -- wave
-    // w copies the K and V rows of kRowsPerWave keys with global_load_lds,
-    // or zeros for an unreadable key -- and the waves read it from there:
-    // two waves per SIMD, one tile each. Two stages, one barrier per step: at
-    // step i a wave waits for its own copies of step i, the barrier
-    // publishes them and frees the stage of step i - 1, which then receives
-    // step i + 1. Rows of the split's keys come from a table filled once per
-    // window of kWindowKeys keys (one page-table load per thread).
-    constexpr int kRowsPerWave = kStepKeys / Sh::kMaxW;
-    static_assert(RPL == 1 && KT == LOADS && kStepKeys % Sh::kMaxW == 0 &&
-                      kWindowKeys % kStepKeys == 0,
-                  "one row per load; whole rows per wave per step");
-    load_q();
-    auto s_kv = reinterpret_cast<uint4 (*)[2][kStepKeys * LPR]>(&s_lds[0]);
-    __shared__ int32_t s_keyrow[kWindowKeys];
-    const uint32_t kv_lds = wave_uniform(lds_address(&s_lds[0]));
-    constexpr uint32_t kRowBytesKV = D * 2;
-    constexpr uint32_t kHalfBytes = kStepKeys * kRowBytesKV;  // K (or V) of one stage
-    const uint64_t kcache = reinterpret_cast<uint64_t>(p.cache_k + (int64_t)head * D);
-    const uint64_t vcache = reinterpret_cast<uint64_t>(p.cache_v + (int64_t)head * D);
-    const uint64_t knew = reinterpret_cast<uint64_t>(p.new_k + ((int64_t)b * c.num_heads + head) * D);
-    const uint64_t vnew = reinterpret_cast<uint64_t>(p.new_v + ((int64_t)b * c.num_heads + head) * D);
-    const uint32_t lane_off = (uint32_t)lane * 16;
-    auto copy_step = [&](int32_t step, int stage) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < kRowsPerWave; ++i) {
-        const int kk = kRowsPerWave * wave + i;
-        const int32_t row = wave_uniform(s_keyrow[step * kStepKeys + kk]);
-        const uint32_t dst = stage * 2 * kHalfBytes + kk * kRowBytesKV;
-        if (row == kRowInvalid) {
-          s_kv[stage][0][kk * LPR + lane] = make_uint4(0, 0, 0, 0);
-          s_kv[stage][1][kk * LPR + lane] = make_uint4(0, 0, 0, 0);
-        } else {
-          const uint64_t off = (uint64_t)(row < 0 ? 0 : row) * Sh::kRowElems * 2;
-          const bool fresh = row == kRowNewToken;
-          copy_row_pair((fresh ? knew : kcache + off) + lane_off, kv_lds + dst);
-          copy_row_pair((fresh ? vnew : vcache + off) + lane_off, kv_lds + dst + kHalfBytes);
-        }
-      }
-    };
-    for (int32_t w0 = 0; w0 < n_keys; w0 += kWindowKeys) {
-      const int32_t wkeys = min(kWindowKeys, n_keys - w0);
-      {
-        const int32_t e = threadIdx.x;
-        const int32_t key = begin + w0 + e;
-        int32_t row = kRowInvalid;
-        if (e < wkeys) {
-          row = key_row(c, p.page_table, p.layer, b, key);
-          row = key == new_pos && row != kRowInvalid ? kRowNewToken : row;
-        }
-        s_keyrow[e] = row;
-      }
-      __syncthreads();
-      const int32_t n_steps = (wkeys + kStepKeys - 1) / kStepKeys;
-      copy_step(0, 0);
-      for (int32_t i = 0; i < n_steps; ++i) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's copies of step i
-        __syncthreads();
-        if (i + 1 < n_steps) copy_step(i + 1, (i + 1) % kStages);
-        const int stage = i % kStages;
-        const int32_t t0 = (i * kLanes + key_lane) * KT;  // first key of my tile
-        TileBuf tb;
-        tb.valid = 0;
-#pragma unroll
-        for (int kl = 0; kl < LOADS; ++kl) {
-          tb.valid |= (s_keyrow[t0 + kl] != kRowInvalid ? 1u : 0u) << kl;
-          tb.k[kl] = s_kv[stage][0][(key_lane * KT + kl) * LPR + cpack];
-          tb.v[kl] = s_kv[stage][1][(key_lane * KT + kl) * LPR + cpack];
-        }
-        compute(tb);
-      }
-      __syncthreads();  // the table and the stages are free for the next window
-    }
-  } else if (my_tiles > 0 && my_tiles <= 2) {
+  if (my_tiles > 0 && my_tiles <= 2) {
     // A wave with one or two tiles (the sliding layers' short splits) runs
     // them straight: the pipeline below would also issue the loads of the
     // dead tiles up to the end of the chunk and wait for them before exit.
@@ -962,64 +641,74 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
 // merged the same way through LDS. Empty splits (l = 0) weigh 0; a row
 // without a live split is zeros.
 constexpr int kCombineThreads = 256;
-// Dims per workgroup: 64 for 256-dim rows (16 split lanes), 32 for 512-dim
+// A batch cut by its lengths (kBalanced) reads its live slots only; over four
+// sequences, 128 dims per workgroup (24 sequences: 6.9 against 26 us with 32,
+// whose 6144 workgroups each derive the cut).
+// Dims per workgroup otherwise: 64 for 256-dim rows (16 split lanes), 32 for 512-dim
 // rows (32 split lanes: the 1 x 512 layer's ~129 splits fold in shorter
 // chains; 24.0 against 24.8 us per layer, while 32 dims for 256-dim rows
 // measured ~1% slower on the per-layer and batch-64 legs).
 template <int kDim>
 constexpr int combine_dims() { return kDim == 512 ? 32 : 64; }
 
-template <int kDim>
-__global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(
-    uint16_t *__restrict__ out, const float *__restrict__ partial_m,
-    const float *__restrict__ partial_l, const float *__restrict__ partial_acc,
-    const int32_t *__restrict__ seq_lengths, int32_t window_size,
-    int32_t split_size, int32_t num_splits, const int32_t *__restrict__ gate) {
-  constexpr int kCombineDims = combine_dims<kDim>();
+template <int kDim, bool kBalanced, int kCombineDims = combine_dims<kDim>()>
+__global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(DecodeParams p) {
   constexpr int kCombineLanes = kCombineThreads / (kCombineDims / 4);  // split lanes
   __shared__ float s_m[kCombineLanes], s_l[kCombineLanes];
   __shared__ float4 s_a[kCombineLanes][kCombineDims / 4];
+  uint16_t *__restrict__ const out = p.out;
+  const int32_t num_splits = p.num_splits;
   const int t = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int dim0 = blockIdx.y * kCombineDims;
-  if (gate != nullptr && *gate != 0) {  // a failed persistent step: zeros
+  if (p.gate != nullptr && *p.gate != 0) {  // a failed persistent step: zeros
     if (t < kCombineDims / 4)
       *reinterpret_cast<uint2 *>(out + row * kDim + dim0 + t * 4) = make_uint2(0, 0);
     return;
   }
   const int32_t b = (int32_t)(row / kQueryHeads);
-  const int32_t seq_word = seq_lengths[b];
+  const int32_t seq_word = p.seq_lengths[b];
 
   const int sl = t / (kCombineDims / 4);  // split lane
   const int dg = t % (kCombineDims / 4);  // 4-dim group
-  const float *pm = partial_m + row * num_splits;
-  const float *pl = partial_l + row * num_splits;
-  const float *pa = partial_acc + row * num_splits * kDim + dim0 + dg * 4;
+  const float *pm = p.partial_m + row * num_splits;
+  const float *pl = p.partial_l + row * num_splits;
+  const float *pa = p.partial_acc + row * num_splits * kDim + dim0 + dg * 4;
   float big_m = -INFINITY, big_l = 0.0f;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  // A batch cut by its lengths: the slots to read follow from them.
+  int32_t cut_splits = 0;
+  if constexpr (kBalanced) {
+    const int32_t keys = lane_live_keys(p);
+    const int32_t splits = balanced_cut(p, keys).splits;
+    cut_splits = __builtin_amdgcn_readlane(keys > 0 ? splits : 0, b);
+  }
+  const int32_t slots = kBalanced ? cut_splits : num_splits;
   // Batches of kBatch split slots per thread: a batch's loads are all issued
   // before its folds, and over every slot up to num_splits, so they do not
   // wait for the length (the empty asm keeps the live-split count, derived
   // from the length, from being computed ahead of them); slots past the
   // live splits were not written this launch and are masked like empty ones.
   constexpr int kBatch = 4;
-  for (int32_t s0 = sl; s0 < num_splits; s0 += kBatch * kCombineLanes) {
+  for (int32_t s0 = sl; s0 < slots; s0 += kBatch * kCombineLanes) {
     float ms_b[kBatch], ls_b[kBatch];
     float4 raw_b[kBatch];
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int32_t s = s0 + i * kCombineLanes;
-      const int32_t slot = s < num_splits ? s : s0;
+      const int32_t slot = s < slots ? s : s0;
       ms_b[i] = pm[slot];
       ls_b[i] = pl[slot];
       raw_b[i] = *reinterpret_cast<const float4 *>(pa + (int64_t)slot * kDim);
     }
     int32_t seq_len = seq_word;
-    asm volatile("" : "+s"(seq_len));
-    int32_t first = window_size > 0 ? seq_len - window_size : 0;
+    asm volatile("" : "+v"(seq_len));
+    seq_len = wave_uniform(seq_len);
+    int32_t first = p.c.window_size > 0 ? seq_len - p.c.window_size : 0;
     first = first < 0 ? 0 : first;
     const int32_t key_count = seq_len > first ? seq_len - first : 0;
-    const int32_t splits = (key_count + split_size - 1) / split_size;
+    const int32_t splits =
+        kBalanced ? cut_splits : (key_count + p.split_size - 1) / p.split_size;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
     const int32_t s = s0 + i * kCombineLanes;
@@ -1072,8 +761,6 @@ __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(
 
 // (8 kv heads x 256): 2 GQA heads per wave, 8 loads -> 16-key tiles.
 using SlidingShape = DecodeShape<8, 256, 2, 8, 2>;
-// (1 kv head x 512): 16 GQA heads as 4 groups of 4, 8 loads -> 8-key tiles.
-using GlobalRefShape = DecodeShape<1, 512, 4, 8, 4, 8>;
 
 bool valid_decode_config(const Gemma4KvCacheConfig &c, int32_t layer) {
   const int64_t capacity = (int64_t)c.max_pages_per_seq * c.page_size;
@@ -1099,7 +786,6 @@ template <class Sh>
 int waves_for(int32_t split_size) {
   const int chunks = (split_size + Sh::CT * Sh::KT - 1) / (Sh::CT * Sh::KT);
   int key_lanes = 1;
-  if constexpr (Sh::kStaged) return Sh::kMaxW;  // two key lanes per head group, always
   // One key lane per started chunk: a split of one chunk stays on one wave
   // (two waves on a 32-key split measured 7.4 against 6.9 us; the merge
   // costs more than the halved tile chain saves).
@@ -1107,22 +793,27 @@ int waves_for(int32_t split_size) {
   return key_lanes * Sh::HG;
 }
 
-template <class Sh>
-hipError_t launch_decode(const DecodeParams &p, int32_t batch_count, bool combine,
-                         hipStream_t stream) {
-  constexpr int D = Sh::LPR * kPackElems;
-  const int waves = waves_for<Sh>(p.split_size);
-  hipLaunchKernelGGL(decode_split_kernel<Sh>,
+hipError_t launch_split_256(const DecodeParams &p, int32_t batch_count, hipStream_t stream) {
+  hipLaunchKernelGGL(decode_split_kernel<SlidingShape>,
                      dim3(p.c.num_heads, p.num_splits, batch_count),
-                     dim3(waves * kWave), 0, stream, p);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !combine || p.num_splits == 1 || p.counters != nullptr) return e;
-  hipLaunchKernelGGL(decode_combine_kernel<D>,
-                     dim3(batch_count * kQueryHeads, D / combine_dims<D>()),
-                     dim3(kCombineThreads), 0, stream, p.out, p.partial_m, p.partial_l,
-                     p.partial_acc, p.seq_lengths, p.c.window_size, p.split_size,
-                     p.num_splits, p.gate);
+                     dim3(waves_for<SlidingShape>(p.split_size) * kWave), 0, stream, p);
   return hipGetLastError();
+}
+
+template <int kDim>
+hipError_t launch_combine(const DecodeParams &p, int32_t batch_count, hipStream_t stream) {
+  auto launch = [&](auto *kernel, int dims) {
+    hipLaunchKernelGGL(kernel, dim3(batch_count * kQueryHeads, kDim / dims), dim3(kCombineThreads),
+                       0, stream, p);
+    return hipGetLastError();
+  };
+  constexpr int kDims = combine_dims<kDim>();
+  if constexpr (kDim == 512) {
+    if (p.balanced != 0 && batch_count > 4)
+      return launch(decode_combine_kernel<kDim, true, 4 * kDims>, 4 * kDims);
+    if (p.balanced != 0) return launch(decode_combine_kernel<kDim, true, kDims>, kDims);
+  }
+  return launch(decode_combine_kernel<kDim, false, kDims>, kDims);
 }
 
 hipError_t decode_entry(uint16_t *out, float *pm, float *pl, float *pacc,
@@ -1174,13 +865,20 @@ hipError_t decode_entry(uint16_t *out, float *pm, float *pl, float *pacc,
   // be numbered by ring slot. A split-only launch hands its partials to the
   // caller in the position-numbered layout.
   p.slot_splits = combine || p.counters != nullptr ? 1 : 0;
-  if (c.num_heads == 8 && c.head_dim == 256) {
-    return launch_decode<SlidingShape>(p, batch_count, combine, stream);
+  // decode_geometry_ok: 8 x 256 or 1 x 512.
+  const bool d512 = c.head_dim == 512;
+  // A batch whose combine follows is cut by its lengths (balanced_cut): two
+  // workgroups per CU, all resident at once.
+  if (d512 && combine && p.counters == nullptr && num_splits > 1 && batch_count >= 2 &&
+      batch_count <= kBalancedBatch) {
+    p.balanced = (int32_t)std::min((int64_t)num_splits * batch_count, (int64_t)kD512Workgroups);
+    p.batch = batch_count;
   }
-  if (c.num_heads == 1 && c.head_dim == 512) {
-    return launch_decode<GlobalRefShape>(p, batch_count, combine, stream);
-  }
-  return hipErrorInvalidValue;
+  const hipError_t e = d512 ? launch_split_d512(p, batch_count, stream)
+                            : launch_split_256(p, batch_count, stream);
+  if (e != hipSuccess || !combine || num_splits == 1 || p.counters != nullptr) return e;
+  return d512 ? launch_combine<512>(p, batch_count, stream)
+              : launch_combine<256>(p, batch_count, stream);
 }
 
 constexpr int kMaxDevices = 64;
@@ -1360,22 +1058,18 @@ hipError_t gemma4_flash_attention_decode_combine_bf16(
       d_partial_l == nullptr || d_partial_acc == nullptr || d_seq_lengths == nullptr) {
     return hipErrorInvalidValue;
   }
-  uint16_t *out = reinterpret_cast<uint16_t *>(d_out);
-  const dim3 block(kCombineThreads);
-  if (config.head_dim == 256) {
-    hipLaunchKernelGGL(decode_combine_kernel<256>, dim3(batch_count * kQueryHeads, 256 / combine_dims<256>()),
-                       block, 0, stream, out, d_partial_m, d_partial_l, d_partial_acc,
-                       d_seq_lengths, config.window_size, split_size, num_splits,
-                       static_cast<const int32_t *>(nullptr));
-  } else if (config.head_dim == 512) {
-    hipLaunchKernelGGL(decode_combine_kernel<512>, dim3(batch_count * kQueryHeads, 512 / combine_dims<512>()),
-                       block, 0, stream, out, d_partial_m, d_partial_l, d_partial_acc,
-                       d_seq_lengths, config.window_size, split_size, num_splits,
-                       static_cast<const int32_t *>(nullptr));
-  } else {
-    return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+  DecodeParams p{};
+  p.out = reinterpret_cast<uint16_t *>(d_out);
+  p.partial_m = const_cast<float *>(d_partial_m);
+  p.partial_l = const_cast<float *>(d_partial_l);
+  p.partial_acc = const_cast<float *>(d_partial_acc);
+  p.seq_lengths = d_seq_lengths;
+  p.c.window_size = config.window_size;
+  p.split_size = split_size;
+  p.num_splits = num_splits;
+  if (config.head_dim == 256) return launch_combine<256>(p, batch_count, stream);
+  if (config.head_dim == 512) return launch_combine<512>(p, batch_count, stream);
+  return hipErrorInvalidValue;
 }
 
 hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
@@ -1391,11 +1085,8 @@ hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
     tile = SlidingShape::KT * SlidingShape::CT;  // one wave's page-lookup chunk
     key_tile = SlidingShape::KT;
   } else if (config.num_heads == 1 && config.head_dim == 512) {
-    // The staged kernel's granule is one LDS step (a tile per key lane):
-    // 8193 keys as 171 splits of 48 run split + combine in 20.5 against
-    // 21.8 us as 129 splits of 64 (32 / 80 / 96 keys: 23.7 / 23.2 / 25.2).
-    tile = (GlobalRefShape::kMaxW / GlobalRefShape::HG) * GlobalRefShape::KT;
-    key_tile = GlobalRefShape::KT;
+    tile = kD512TileKeys;
+    key_tile = kD512TileKeys / 2;
   } else {
     return hipErrorInvalidValue;
   }
@@ -1414,6 +1105,9 @@ hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
   int64_t size = (keys + splits_per_seq - 1) / splits_per_seq;
   size = ((size + tile - 1) / tile) * tile;
   if (size < tile) size = tile;
+  // Shorter splits of a 1 x 512 batch pay more for their start than they
+  // spread the work; the launch lengthens them to fit the chip (balanced_cut).
+  if (planned && config.head_dim == 512 && batch_count > 1) size = std::max<int64_t>(size, kD512BatchSplit);
   // One sequence whose splits come out at two tiles or fewer (a sliding
   // layer's 1024-key window): the split is a dependent chain of tile
   // latencies, so one tile per workgroup, as long as that stays within two

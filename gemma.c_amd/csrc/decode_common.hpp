@@ -39,6 +39,11 @@ struct DecodeParams {
   // Nonzero: a full ring may be split by ring slot rather than by position
   // (the partials are internal to the launch).
   int32_t slot_splits = 0;
+  // Nonzero (1 x 512, 2 .. 64 sequences, partials internal to the launch):
+  // sequences are cut by their lengths, see balanced_cut. The value is the
+  // number of split workgroups, batch the number of sequences.
+  int32_t balanced = 0;
+  int32_t batch = 0;
 };
 
 constexpr int kRowInvalid = -1;   // key outside the split or unmapped page
@@ -203,6 +208,70 @@ __device__ __forceinline__ auto coherent_view(const float *p, int32_t count) {
 // batch and split plan (the checks decode_entry makes before any launch).
 bool decode_geometry_ok(const Gemma4KvCacheConfig &c, int32_t layer, int32_t batch_count,
                         int32_t split_size, int32_t num_splits);
+
+// 1 x 512 split kernel (decode_d512.hip).
+constexpr int kD512TileKeys = 16;     // keys of a wave's tile
+constexpr int kD512Workgroups = 512;  // balanced: two 69 KiB workgroups on each of 256 CUs
+// The plan's shortest split of a batch. 64 / 96 / 128 keys: 2 x 8193 20.9 / 18.9 /
+// 20.4 us, 8 x 100-4000 20.4 / 18.7 / 19.6 us, 16 x 30-1200 16.7 / 17.9 / 19.2 us.
+constexpr int kD512BatchSplit = 96;
+
+// Splits of a batch cut on the device, by the lengths that only it knows. One
+// split size for every sequence, the smallest multiple of kBalancedStep keys
+// (and no less than the plan's, so that the plan's partial slots suffice) for
+// which all splits run at once: sum of ceil(len / size) <= workgroups, by
+// size >= total / (workgroups - batch). Measured, split + combine: 24 sequences
+// of 200-12001 keys 62 us (fixed splits of 96 / 192 / 512 keys: 95 / 83 / 80,
+// the workgroups of the plan's dead splits and the last, part-filled round
+// being what they lose), 3 of 400-90000 51 us (74 / 62 / 59), 64 of 100-4500
+// 72 us (126 / 126 / 107). A sequence has one split at least
+// (which appends its token). Lane i of every wave calls this with sequence
+// i's live key count (0 for i >= batch).
+constexpr int kBalancedBatch = kWave;
+constexpr int kBalancedStep = kD512TileKeys;
+struct BalancedCut {
+  int32_t size;    // keys per split
+  int32_t splits;  // of this lane's sequence (0 past the batch)
+};
+__device__ __forceinline__ BalancedCut balanced_cut(const DecodeParams &p, int32_t keys) {
+  const int lane = __lane_id();
+  // The plan's slots bound what a sequence can hold, as with fixed splits.
+  const int64_t capacity = (int64_t)p.split_size * p.num_splits;
+  const uint32_t held = (uint32_t)min((int64_t)keys, capacity);
+  uint32_t size = (uint32_t)p.split_size;
+  if ((int64_t)p.num_splits * p.batch > p.balanced) {
+    // Sums of the low and high halves: 64 keys counts below 2^31 each.
+    uint32_t lo = held & 0xFFFFu, hi = held >> 16;
+#pragma unroll
+    for (int mask = 1; mask < kWave; mask *= 2) {
+      lo += __shfl_xor(lo, mask);
+      hi += __shfl_xor(hi, mask);
+    }
+    const uint64_t total = ((uint64_t)hi << 16) + lo;
+    const uint32_t room = (uint32_t)(p.balanced - p.batch);  // > 0: see the launch
+    // One 32-bit division in any real cache; the long one is a branch.
+    const uint64_t even = total < 0x80000000u ? ((uint32_t)total + room - 1) / room
+                                              : (total + room - 1) / room;
+    const uint32_t rounded = ((uint32_t)even + kBalancedStep - 1) & ~(uint32_t)(kBalancedStep - 1);
+    size = max(size, rounded);
+  }
+  BalancedCut cut;
+  cut.size = wave_uniform((int32_t)size);
+  cut.splits = lane < p.batch ? max(1, (int32_t)((held + size - 1) / size)) : 0;
+  return cut;
+}
+// Live keys of sequence `lane` of the batch (0 past it).
+__device__ __forceinline__ int32_t lane_live_keys(const DecodeParams &p) {
+  const int lane = __lane_id();
+  const int32_t len = p.seq_lengths[lane < p.batch ? lane : 0];
+  const int32_t first = p.c.window_size > 0 ? max(len - p.c.window_size, 0) : 0;
+  return lane < p.batch && len > first ? len - first : 0;
+}
+
+
+// Split phase of the 1 x 512 geometry (decode_d512.hip) on a grid of
+// (p.num_splits, batch_count); checked arguments.
+hipError_t launch_split_d512(const DecodeParams &p, int32_t batch_count, hipStream_t stream);
 
 // The fused append + split-K decode with the separate combine
 // (decode_attention.hip) for the persistent step's 1 x 512 global layers:

@@ -31,6 +31,15 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
 }
 
+// The same pair by the hardware conversion (v_cvt_pk_bf16_f32): round to
+// nearest even, NaN stays NaN; one instruction for the ~15 of pack_bf16x2.
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
+  const f32x2_t f = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
+}
+
 __device__ __forceinline__ uint4 load128(const void *p) {
   return *reinterpret_cast<const uint4 *>(p);
 }
@@ -55,7 +64,6 @@ __device__ __forceinline__ void unpack8(const uint4 &p, float (&f)[8]) {
 
 // a.lo*b.lo + a.hi*b.hi + c for packed bf16 pairs (v_dot2c_f32_bf16): the
 // products are exact in fp32 and the sum is rounded once per step.
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a),
                                         __builtin_bit_cast(bf16x2_t, b), c, false);

@@ -36,6 +36,7 @@ HIP_FLAGS = [
 # allocator copies all 128 accumulators between AGPRs and VGPRs on every tile
 # to serve that path, so their MFMAs are selected in the VGPR form.
 EXTRA_FLAGS = {
+    "decode_d512": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
     "prefill_attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
     "prefill_norm_rope": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
 }

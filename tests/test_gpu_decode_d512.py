@@ -1,0 +1,113 @@
+"""The 1 x 512 split kernel (decode_d512.hip) against the oracle at the sizes
+where it can go wrong: splits of one key to several steps of both workgroup
+forms (a step is 16 keys per wave), ragged last tiles, idle waves, page
+lookups past the first four steps, rings, unmapped pages, and batches whose
+splits the device cuts by the lengths (more planned splits than workgroups).
+Cache rows that no sequence may read hold NaN: a value that leaks through a
+masked key shows."""
+import math
+
+import numpy as np
+import pytest
+
+from kvtest import assert_close, cache_config, fill_page_table, from_dev_bf16, randn_bf16, ring_pages, to_dev
+from oracle import oracle
+from test_gpu_decode import _run_decode
+
+pytestmark = pytest.mark.gpu
+NAN = np.uint16(0x7FC0)
+
+# (split size, lengths, window, page)
+CASES = [
+    (1, [3], 0, 16),
+    (15, [31], 0, 16),
+    (16, [33], 0, 1),
+    (48, [8, 97], 0, 16),              # cut by length: 2 x 3 slots, all run
+    (63, [64, 127, 190], 0, 64),
+    (64, [1, 64, 65], 0, 16),
+    (65, [66], 0, 16),                 # two-wave form: a step and one key
+    (96, [95, 96, 97, 0, 300], 0, 64),
+    (160, [159, 161], 0, 16),          # past four steps: the second page lookup
+    (333, [1000], 0, 16),
+    (512, [512], 0, 64),               # a single split, written directly
+    (40, [500], 256, 16),              # a ring, split by position
+    (70, [80, 256, 700], 256, 1),
+    (16, [4001, 17, 2900], 0, 64),     # 753 planned splits on 512 workgroups
+    (16, [11 * i for i in range(64)], 0, 16),
+    (16, [9 * i for i in range(65)], 0, 16),  # past the batch that is cut by length
+]
+
+
+def _case(rng, split, seq, window, page):
+    batch = len(seq)
+    max_pages = ring_pages(window, page) if window else max(1, -(-max(seq) // page))
+    cfg = cache_config(1, batch, page, max_pages, 1, 512, window)
+    pt = fill_page_table(cfg, seq)
+    rows = batch * max_pages * page
+    ck, cv = np.full((rows, 1, 512), NAN), np.full((rows, 1, 512), NAN)
+    for b, n in enumerate(seq):
+        pos = np.arange(max(0, n - window) if window else 0, n)
+        r = pt[b * max_pages + (pos // page) % max_pages].astype(np.int64) * page + pos % page
+        ck[r], cv[r] = randn_bf16(rng, (len(r), 1, 512)), randn_bf16(rng, (len(r), 1, 512))
+    live = max(min(n, window) if window else n for n in seq)
+    return cfg, pt, ck, cv, randn_bf16(rng, (batch, 16, 512)), -(-live // split)
+
+
+@pytest.mark.parametrize("split,seq,window,page", CASES)
+def test_split_sizes(dev, split, seq, window, page):
+    rng = np.random.default_rng(split * 1000 + len(seq))
+    cfg, pt, ck0, cv0, q, splits = _case(rng, split, seq, window, page)
+    print(f"split {split}x{splits} seq {seq[:6]} window {window} page {page}", flush=True)
+    scale = 1.0 / math.sqrt(512)
+    # The token of the last position; a sequence without keys has none.
+    k, v = randn_bf16(rng, (len(seq), 1, 512)), randn_bf16(rng, (len(seq), 1, 512))
+    pos = [n - 1 for n in seq]
+    exp_k, exp_v = ck0.copy(), cv0.copy()
+    oracle.kv_cache_write(exp_k, exp_v, cfg, pt, list(range(len(seq))), pos, 0, k, v)
+    exp = oracle.decode_attention(q, exp_k, exp_v, pt, seq, cfg, 0, scale)
+    ck, cv = to_dev(ck0, dev), to_dev(cv0, dev)
+    got = _run_decode(dev, cfg, q, ck, cv, pt, seq, 0, scale, split, splits, fused=(pos, k, v))
+    assert np.array_equal(from_dev_bf16(ck).reshape(exp_k.shape), exp_k)
+    assert np.array_equal(from_dev_bf16(cv).reshape(exp_v.shape), exp_v)
+    assert_close(got, exp, "appended")
+    # The same without an append, over the cache it left.
+    got = _run_decode(dev, cfg, q, ck, cv, pt, seq, 0, scale, split, splits)
+    assert_close(got, exp, "no append")
+
+
+def test_unmapped_pages_in_a_batch(dev):
+    """Unmapped pages inside the live range, among them the token's own."""
+    rng = np.random.default_rng(77)
+    seq = [200, 90, 333]
+    cfg, pt, ck0, cv0, q, splits = _case(rng, 16, seq, 0, 16)
+    max_pages = cfg[3]
+    pt[3] = pt[max_pages + 5] = pt[2 * max_pages + 20] = -1  # page 5 holds position 89
+    k, v = randn_bf16(rng, (3, 1, 512)), randn_bf16(rng, (3, 1, 512))
+    pos = [n - 1 for n in seq]
+    exp_k, exp_v = ck0.copy(), cv0.copy()
+    oracle.kv_cache_write(exp_k, exp_v, cfg, pt, [0, 1, 2], pos, 0, k, v)
+    exp = oracle.decode_attention(q, exp_k, exp_v, pt, seq, cfg, 0, 0.0442)
+    ck, cv = to_dev(ck0, dev), to_dev(cv0, dev)
+    got = _run_decode(dev, cfg, q, ck, cv, pt, seq, 0, 0.0442, 16, splits, fused=(pos, k, v))
+    assert np.array_equal(from_dev_bf16(ck).reshape(exp_k.shape), exp_k)
+    assert_close(got, exp, "unmapped")
+
+
+def test_token_outside_the_live_keys_is_appended(dev):
+    """A token past its sequence's length (also an empty one) is stored and
+    not attended to, in a batch cut by its lengths."""
+    rng = np.random.default_rng(78)
+    held = [40, 16, 600]
+    cfg, pt, ck0, cv0, q, _ = _case(rng, 16, held, 0, 16)
+    seq = [20, 0, 599]
+    k, v = randn_bf16(rng, (3, 1, 512)), randn_bf16(rng, (3, 1, 512))
+    pos = [33, 4, 599]
+    exp = oracle.decode_attention(q, ck0, cv0, pt, seq, cfg, 0, 0.05)
+    exp_k, exp_v = ck0.copy(), cv0.copy()
+    oracle.kv_cache_write(exp_k, exp_v, cfg, pt, [0, 1, 2], pos, 0, k, v)
+    ck, cv = to_dev(ck0, dev), to_dev(cv0, dev)
+    got = _run_decode(dev, cfg, q, ck, cv, pt, seq, 0, 0.05, 16, 38, fused=(pos, k, v))
+    assert np.array_equal(from_dev_bf16(ck).reshape(exp_k.shape), exp_k)
+    assert np.array_equal(from_dev_bf16(cv).reshape(exp_v.shape), exp_v)
+    assert_close(got, exp, "outside")
+    assert not got[1].any()
