@@ -868,9 +868,11 @@ hipError_t decode_entry(uint16_t *out, float *pm, float *pl, float *pacc,
   // decode_geometry_ok: 8 x 256 or 1 x 512.
   const bool d512 = c.head_dim == 512;
   // A batch whose combine follows is cut by its lengths (balanced_cut): two
-  // workgroups per CU, all resident at once.
-  if (d512 && combine && p.counters == nullptr && num_splits > 1 && batch_count >= 2 &&
-      batch_count <= kBalancedBatch) {
+  // workgroups per CU, all resident at once. One sequence is planned by its
+  // length already, except in a step (gate), which plans by the cache's
+  // capacity: a cut there once that gives splits of more than one step.
+  if (d512 && combine && p.counters == nullptr && num_splits > 1 && batch_count <= kBalancedBatch &&
+      (batch_count >= 2 || (gate != nullptr && split_size > 4 * kD512TileKeys))) {
     p.balanced = (int32_t)std::min((int64_t)num_splits * batch_count, (int64_t)kD512Workgroups);
     p.batch = batch_count;
   }

@@ -39,7 +39,7 @@ struct DecodeParams {
   // Nonzero: a full ring may be split by ring slot rather than by position
   // (the partials are internal to the launch).
   int32_t slot_splits = 0;
-  // Nonzero (1 x 512, 2 .. 64 sequences, partials internal to the launch):
+  // Nonzero (1 x 512, up to 64 sequences, partials internal to the launch):
   // sequences are cut by their lengths, see balanced_cut. The value is the
   // number of split workgroups, batch the number of sequences.
   int32_t balanced = 0;
@@ -217,16 +217,17 @@ constexpr int kD512Workgroups = 512;  // balanced: two 69 KiB workgroups on each
 constexpr int kD512BatchSplit = 96;
 
 // Splits of a batch cut on the device, by the lengths that only it knows. One
-// split size for every sequence, the smallest multiple of kBalancedStep keys
-// (and no less than the plan's, so that the plan's partial slots suffice) for
-// which all splits run at once: sum of ceil(len / size) <= workgroups, by
-// size >= total / (workgroups - batch). Measured, split + combine: 24 sequences
-// of 200-12001 keys 62 us (fixed splits of 96 / 192 / 512 keys: 95 / 83 / 80,
-// the workgroups of the plan's dead splits and the last, part-filled round
-// being what they lose), 3 of 400-90000 51 us (74 / 62 / 59), 64 of 100-4500
-// 72 us (126 / 126 / 107). A sequence has one split at least
-// (which appends its token). Lane i of every wave calls this with sequence
-// i's live key count (0 for i >= batch).
+// split size for every sequence: the smallest multiple of kBalancedStep keys,
+// kD512BatchSplit at least, that fits the plan's partial slots
+// (ceil(longest / size) <= num_splits) and lets all splits run at once
+// (sum of ceil(len / size) <= workgroups, by size >= total / (workgroups -
+// batch)). The plan knows only a longest length, often a cache's capacity.
+// Measured, split + combine: 24 sequences of 200-12001 keys 62 us (fixed
+// splits of 96 / 192 / 512 keys: 95 / 83 / 80, the workgroups of the plan's
+// dead splits and the last, part-filled round being what they lose), 3 of
+// 400-90000 51 us (74 / 62 / 59), 64 of 100-4500 72 us (126 / 126 / 107). A
+// sequence has one split at least (which appends its token). Lane i of every
+// wave calls this with sequence i's live key count (0 for i >= batch).
 constexpr int kBalancedBatch = kWave;
 constexpr int kBalancedStep = kD512TileKeys;
 struct BalancedCut {
@@ -238,22 +239,26 @@ __device__ __forceinline__ BalancedCut balanced_cut(const DecodeParams &p, int32
   // The plan's slots bound what a sequence can hold, as with fixed splits.
   const int64_t capacity = (int64_t)p.split_size * p.num_splits;
   const uint32_t held = (uint32_t)min((int64_t)keys, capacity);
-  uint32_t size = (uint32_t)p.split_size;
-  if ((int64_t)p.num_splits * p.batch > p.balanced) {
-    // Sums of the low and high halves: 64 keys counts below 2^31 each.
-    uint32_t lo = held & 0xFFFFu, hi = held >> 16;
+  // The longest, and sums of the low and high halves (64 counts below 2^31).
+  uint32_t longest = held, lo = held & 0xFFFFu, hi = held >> 16;
 #pragma unroll
-    for (int mask = 1; mask < kWave; mask *= 2) {
-      lo += __shfl_xor(lo, mask);
-      hi += __shfl_xor(hi, mask);
-    }
+  for (int mask = 1; mask < kWave; mask *= 2) {
+    longest = max(longest, (uint32_t)__shfl_xor(longest, mask));
+    lo += __shfl_xor(lo, mask);
+    hi += __shfl_xor(hi, mask);
+  }
+  auto whole_steps = [](uint32_t n) {
+    return (n + kBalancedStep - 1) & ~(uint32_t)(kBalancedStep - 1);
+  };
+  const uint32_t slots = (uint32_t)p.num_splits;
+  uint32_t size = max((uint32_t)kD512BatchSplit, whole_steps((longest + slots - 1) / slots));
+  if ((int64_t)p.num_splits * p.batch > p.balanced) {
     const uint64_t total = ((uint64_t)hi << 16) + lo;
     const uint32_t room = (uint32_t)(p.balanced - p.batch);  // > 0: see the launch
     // One 32-bit division in any real cache; the long one is a branch.
     const uint64_t even = total < 0x80000000u ? ((uint32_t)total + room - 1) / room
                                               : (total + room - 1) / room;
-    const uint32_t rounded = ((uint32_t)even + kBalancedStep - 1) & ~(uint32_t)(kBalancedStep - 1);
-    size = max(size, rounded);
+    size = max(size, whole_steps((uint32_t)even));
   }
   BalancedCut cut;
   cut.size = wave_uniform((int32_t)size);

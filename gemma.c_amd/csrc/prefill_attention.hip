@@ -52,6 +52,7 @@
 
 #include "gemma4_flash_attention.h"
 
+#include <algorithm>
 #include <math.h>
 
 #include <type_traits>
@@ -92,7 +93,13 @@ struct PrefillParams {
   // pair splits meets in its slot of the workspace.
   int32_t n_pairs;
   char *ws;
+  // Chunks of few row blocks (n_parts > 1): every row block's key tiles are
+  // shared out over up to n_parts workgroups, whose partials a second launch
+  // merges.
+  int32_t n_parts;
 };
+
+enum class Mode { kPlain, kPaired, kParts };
 
 constexpr int kPartialFloats = 130;  // per thread: 128 accumulators, max, sum
 // Workspace slot s at s * kSlotBytes: the arrival counter (256-byte
@@ -100,7 +107,23 @@ constexpr int kPartialFloats = 130;  // per thread: 128 accumulators, max, sum
 // each, element-major). A slot sits at the same place for every chunk
 // length, so calls of different sizes can share a workspace.
 constexpr int64_t kSlotCounterBytes = 256;
-constexpr int64_t kSlotBytes = kSlotCounterBytes + 2LL * kPartialFloats * kPrefillThreads * 4;
+constexpr int64_t kPartialBytes = (int64_t)kPartialFloats * kPrefillThreads * 4;
+constexpr int64_t kSlotBytes = kSlotCounterBytes + 2LL * kPartialBytes;
+// Partial i of a chunk in parts: half i % 2 of slot i / 2, so that a balanced
+// chunk that uses the same workspace later finds its counters untouched.
+__device__ __forceinline__ float *part_partial(char *ws, int64_t i) {
+  return reinterpret_cast<float *>(ws + (i >> 1) * kSlotBytes + kSlotCounterBytes +
+                                   (i & 1) * kPartialBytes);
+}
+// A row block's share of `tiles` key tiles in parts: tiles per part, two at
+// least (a workgroup's start costs as much as five tiles).
+__device__ __forceinline__ int part_tiles(int tiles, int n_parts) {
+  return max((tiles + n_parts - 1) / n_parts, 2);
+}
+// Key tiles of causal row block blk (no window).
+__device__ __forceinline__ int causal_tiles(int prior, int chunk_len, int blk) {
+  return (prior + min(kPrefillRows * (blk + 1), chunk_len) - 1) / kTileKeys + 1;
+}
 
 __device__ __forceinline__ f32x16_t mfma32(uint4 a, uint4 b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
@@ -190,7 +213,7 @@ __device__ __forceinline__ void static_for(F &&f) {
 template <int kSt>
 using Stage = std::integral_constant<int, kSt>;
 
-template <bool kPaired>
+template <Mode kMode>
 __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(PrefillParams p) {
   constexpr int KS = kDim / 16;        // k-steps of S^T (dims)
   constexpr int DB = kDim / 32;        // 32-dim blocks of O^T
@@ -240,14 +263,24 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   constexpr int kAllTiles = 1 << 30;
   Unit unit0 = {0, 0, 0, -1, 0}, unit1 = {0, 0, 0, -1, 0};
   int n_units = 0;
-  if constexpr (kPaired) {
+  int part = 0, live_parts = 1;
+  if constexpr (kMode == Mode::kParts) {
+    const int rest = blockIdx.x / Hk;
+    const int blk = rest / p.n_parts;
+    part = rest % p.n_parts;
+    const int tiles = causal_tiles(prior, Lq, blk);
+    const int per = part_tiles(tiles, p.n_parts);
+    live_parts = (tiles + per - 1) / per;
+    if (part >= live_parts) return;
+    unit0 = {kPrefillRows * blk, part * per, part == live_parts - 1 ? kAllTiles : (part + 1) * per,
+             -1, 0};
+    n_units = 1;
+  } else if constexpr (kMode == Mode::kPaired) {
     const int rest = blockIdx.x / Hk;
     const int pair = rest >> 1, side = rest & 1;
     const int nb = (Lq + kPrefillRows - 1) / kPrefillRows;
     const int j = pair, J = nb - 1 - pair;
-    auto tiles_of = [&](int blk) {  // causal, no window: tiles 0 .. last key
-      return (prior + min(kPrefillRows * (blk + 1), Lq) - 1) / kTileKeys + 1;
-    };
+    auto tiles_of = [&](int blk) { return causal_tiles(prior, Lq, blk); };
     if (j == J) {
       if (side == 0) {
         unit0 = {kPrefillRows * j, 0, kAllTiles, -1, 0};
@@ -625,6 +658,22 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   // other half may run on another XCD), count the arrival, and let the
   // second arriver merge both halves and write the rows.
   bool emit = true;
+  if (kMode == Mode::kParts && live_parts > 1) {
+    // Rows past the chunk are not merged and need no partial.
+    emit = false;
+    if (row_ok) {
+      const int nb = (Lq + kPrefillRows - 1) / kPrefillRows;
+      float *mine = part_partial(
+          p.ws, (((int64_t)b * nb + q0 / kPrefillRows) * Hk + head) * p.n_parts + part);
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mine[(d * 16 + i) * kPrefillThreads + t] = acc[d][i];
+      }
+      mine[128 * kPrefillThreads + t] = m_run;
+      mine[129 * kPrefillThreads + t] = l_run;
+    }
+  }
   if (unit_slot >= 0) {
     char *slot = p.ws + (int64_t)unit_slot * kSlotBytes;
     float *part = reinterpret_cast<float *>(slot + kSlotCounterBytes);
@@ -696,8 +745,71 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
       }
     }
   }
-  if constexpr (kPaired) __syncthreads();  // the next unit reuses the LDS stages and tables
+  if constexpr (kMode == Mode::kPaired) __syncthreads();  // the next unit reuses the LDS stages and tables
   }  // units
+}
+
+// Merges the parts of a chunk's row blocks: workgroup (kv head, row block,
+// slice of 8 of a thread's 128 accumulators), thread t as in the chunk kernel.
+constexpr int kMergeElems = 8;
+constexpr int kMergeSlices = 128 / kMergeElems;
+__global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillParams p) {
+  const int t = threadIdx.x;
+  const int lane = t & 63, wave = t >> 6;
+  const int Hk = p.c.num_heads;
+  const int head = blockIdx.x % Hk;
+  const int blk = blockIdx.x / Hk / kMergeSlices;
+  const int e0 = blockIdx.x / Hk % kMergeSlices * kMergeElems;
+  const int b = blockIdx.y;
+  const int Lq = p.chunk_len;
+  const int prior = p.prior != nullptr ? wave_uniform(p.prior[b]) : 0;
+  const int tiles = causal_tiles(prior, Lq, blk);
+  const int per = part_tiles(tiles, p.n_parts);
+  const int live_parts = (tiles + per - 1) / per;
+  if (live_parts == 1) return;  // the chunk kernel wrote the rows
+  const int nb = (Lq + kPrefillRows - 1) / kPrefillRows;
+  const int n = lane & 31, half = lane >> 5;
+  const int row = blk * kPrefillRows + 16 * wave + n % 16;
+  if (row >= Lq) return;
+  const int64_t part0 = (((int64_t)b * nb + blk) * Hk + head) * p.n_parts;
+  float m = -INFINITY, l = 0.0f;
+  float acc[kMergeElems] = {};
+  constexpr int kBatch = 4;  // parts whose loads go out together
+  for (int i0 = 0; i0 < live_parts; i0 += kBatch) {
+    float pm[kBatch], pl[kBatch], pa[kBatch][kMergeElems];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const float *part = part_partial(p.ws, part0 + min(i0 + i, live_parts - 1)) + t;
+      pm[i] = part[128 * kPrefillThreads];
+      pl[i] = part[129 * kPrefillThreads];
+#pragma unroll
+      for (int e = 0; e < kMergeElems; ++e) pa[i][e] = part[(e0 + e) * kPrefillThreads];
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const float mi = i0 + i < live_parts ? pm[i] : -INFINITY;
+      const float m_new = fmaxf(m, mi);
+      const float fa = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+      const float fb = mi == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mi - m_new);
+      l = l * fa + pl[i] * fb;
+#pragma unroll
+      for (int e = 0; e < kMergeElems; ++e) acc[e] = acc[e] * fa + pa[i][e] * fb;
+      m = m_new;
+    }
+  }
+  // Lanes l and l ^ 32 hold one row's sums over different keys (and share
+  // the maximum). Both are here: they have the same row.
+  l = xor_sum<32>(l);
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const int qh = head * (kQueryHeads / Hk) + n / 16;
+  uint16_t *orow = p.out + (((int64_t)b * Lq + row) * kQueryHeads + qh) * kDim;
+#pragma unroll
+  for (int i = 0; i < kMergeElems; i += 4) {
+    const int d = (e0 + i) / 16, ii = (e0 + i) % 16;
+    *reinterpret_cast<uint2 *>(orow + 32 * d + (ii / 4) * 8 + 4 * half) =
+        make_uint2(pack_bf16x2(acc[i] * inv, acc[i + 1] * inv),
+                   pack_bf16x2(acc[i + 2] * inv, acc[i + 3] * inv));
+  }
 }
 
 }  // namespace
@@ -717,6 +829,30 @@ size_t prefill_workspace_bytes(int32_t batch_size, int32_t chunk_len, int32_t he
   if (batch_size <= 0 || chunk_len <= 0 || heads <= 0) return 0;
   const int64_t slots = (int64_t)batch_size * heads * prefill_pairs(chunk_len);
   return (size_t)(slots * kSlotBytes);
+}
+
+// Parts per row block for a global chunk that leaves half of the 256 CUs or
+// more without a row block: as many as give every CU a workgroup, if the
+// cache (or the chunk) has room for enough keys to be worth the second
+// launch; the lengths are on the device. 93 rows after 7401 tokens: 254 -> 33 us (in
+// 15 parts of 8 tiles: the chunk launch 27, the merge 6.5).
+constexpr int kPartsCus = 256;
+constexpr int kPartsMinTiles = 6;
+bool parts_worthwhile(int32_t chunk_len, const Gemma4KvCacheConfig &c) {
+  const int64_t capacity = c.max_pages_per_seq > 0 && c.page_size > 0
+                               ? (int64_t)c.max_pages_per_seq * c.page_size : 0;
+  return c.window_size == 0 &&
+         std::max<int64_t>(capacity, chunk_len) >= kPartsMinTiles * kTileKeys;
+}
+int64_t row_blocks(int32_t batch_size, int32_t chunk_len, int32_t heads) {
+  return (int64_t)batch_size * heads * ((chunk_len + kPrefillRows - 1) / kPrefillRows);
+}
+// Parts that `workspace_bytes` hold, 1 if the form does not apply.
+int prefill_parts(int32_t batch_size, int32_t chunk_len, const Gemma4KvCacheConfig &c,
+                  size_t workspace_bytes) {
+  if (!parts_worthwhile(chunk_len, c)) return 1;
+  const int64_t held = std::min<int64_t>(kPartsCus, 2 * (int64_t)(workspace_bytes / kSlotBytes));
+  return (int)std::max<int64_t>(1, held / row_blocks(batch_size, chunk_len, c.num_heads));
 }
 
 hipError_t prefill_chunk_launch(gemma4_bf16 *d_out, const gemma4_bf16 *d_q, const gemma4_bf16 *d_k,
@@ -744,7 +880,7 @@ hipError_t prefill_chunk_launch(gemma4_bf16 *d_out, const gemma4_bf16 *d_q, cons
                    (reinterpret_cast<uintptr_t>(d_workspace) & 255) != 0)) {
     return hipErrorInvalidValue;
   }
-  PrefillParams p;
+  PrefillParams p{};
   p.out = reinterpret_cast<uint16_t *>(d_out);
   p.q = reinterpret_cast<const uint16_t *>(d_q);
   p.k = reinterpret_cast<const uint16_t *>(d_k);
@@ -766,14 +902,28 @@ hipError_t prefill_chunk_launch(gemma4_bf16 *d_out, const gemma4_bf16 *d_q, cons
   // Sliding chunks already carry equal work per row block; only causal
   // (global) chunks of two or more row blocks are paired.
   p.n_pairs = balanced && config.window_size == 0 ? prefill_pairs(chunk_len) : 0;
-  p.ws = p.n_pairs > 0 ? static_cast<char *>(d_workspace) : nullptr;
-  int blocks = config.num_heads * ((chunk_len + kPrefillRows - 1) / kPrefillRows);
-  if (p.n_pairs > 0) blocks = config.num_heads * 2 * p.n_pairs;
-  if (p.n_pairs > 0) {
-    hipLaunchKernelGGL(prefill_chunk_kernel<true>, dim3(blocks, batch_size),
+  p.ws = static_cast<char *>(d_workspace);
+  const int blocks = (int)row_blocks(1, chunk_len, config.num_heads);
+  // In parts as far as the caller's workspace goes (one sized before this
+  // form, or none for a single row block, serves the forms below).
+  const bool usable =
+      d_workspace != nullptr && (reinterpret_cast<uintptr_t>(d_workspace) & 255) == 0;
+  const int parts =
+      usable ? prefill_parts(batch_size, chunk_len, config, workspace_bytes) : 1;
+  if (parts > 1) {
+    p.n_parts = parts;
+    hipLaunchKernelGGL(prefill_chunk_kernel<Mode::kParts>, dim3(blocks * parts, batch_size),
                        dim3(kPrefillThreads), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(prefill_merge_kernel, dim3(blocks * kMergeSlices, batch_size),
+                       dim3(kPrefillThreads), 0, stream, p);
+  } else if (p.n_pairs > 0) {
+    hipLaunchKernelGGL(prefill_chunk_kernel<Mode::kPaired>,
+                       dim3(config.num_heads * 2 * p.n_pairs, batch_size), dim3(kPrefillThreads), 0,
+                       stream, p);
   } else {
-    hipLaunchKernelGGL(prefill_chunk_kernel<false>, dim3(blocks, batch_size),
+    hipLaunchKernelGGL(prefill_chunk_kernel<Mode::kPlain>, dim3(blocks, batch_size),
                        dim3(kPrefillThreads), 0, stream, p);
   }
   return hipGetLastError();
@@ -794,8 +944,12 @@ extern "C" hipError_t gemma4_flash_attention_prefill_chunk_paged_bf16(
 
 extern "C" size_t gemma4_flash_attention_prefill_chunk_workspace_bytes(
     int32_t batch_size, int32_t chunk_len, Gemma4KvCacheConfig config) {
-  return config.window_size == 0 ? prefill_workspace_bytes(batch_size, chunk_len, config.num_heads)
-                                 : 0;
+  if (config.window_size != 0 || batch_size <= 0 || chunk_len <= 0 || config.num_heads <= 0)
+    return 0;
+  // For every chunk length and batch alike, so that a workspace sized for the
+  // largest serves all.
+  const size_t parts = parts_worthwhile(chunk_len, config) ? kPartsCus / 2 * kSlotBytes : 0;
+  return std::max(prefill_workspace_bytes(batch_size, chunk_len, config.num_heads), parts);
 }
 
 extern "C" hipError_t gemma4_flash_attention_prefill_chunk_paged_bf16_ws(

@@ -161,7 +161,8 @@ hipError_t gemma4_flash_attention_prefill_chunk_paged_bf16(
 // up to float summation order. d_workspace: at least
 // gemma4_flash_attention_prefill_chunk_workspace_bytes(batch_size,
 // chunk_len, config) bytes, 256-byte aligned, zero-filled once before its
-// first use (every call leaves its arrival counters at zero again); one
+// first use (every call leaves its arrival counters at zero again; a
+// single row block may also come without one); one
 // sized for the largest chunk and batch also serves every smaller call;
 // calls that share a workspace must not overlap. Sliding chunks (window > 0) run
 // the plain kernel and ignore the workspace. No counterpart in the

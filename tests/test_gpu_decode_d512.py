@@ -10,6 +10,7 @@ import math
 import numpy as np
 import pytest
 
+import gemma_kv as gk
 from kvtest import assert_close, cache_config, fill_page_table, from_dev_bf16, randn_bf16, ring_pages, to_dev
 from oracle import oracle
 from test_gpu_decode import _run_decode
@@ -111,3 +112,42 @@ def test_token_outside_the_live_keys_is_appended(dev):
     assert np.array_equal(from_dev_bf16(cv).reshape(exp_v.shape), exp_v)
     assert_close(got, exp, "outside")
     assert not got[1].any()
+
+
+def test_plan_longer_than_the_lengths(dev):
+    """Splits of a plan made for 4000 keys over sequences of 31 to 700: the
+    device's cut is finer than the plan's."""
+    rng = np.random.default_rng(79)
+    seq = [150, 700, 31]
+    cfg, pt, ck0, cv0, q, _ = _case(rng, 16, seq, 0, 16)
+    exp = oracle.decode_attention(q, ck0, cv0, pt, seq, cfg, 0, 0.05)
+    got = _run_decode(dev, cfg, q, to_dev(ck0, dev), to_dev(cv0, dev), pt, seq, 0, 0.05, 200, 20)
+    assert_close(got, exp, "finer cut")
+
+
+def test_step_plans_by_capacity(dev):
+    """A step's global layer over a cache far larger than its sequence (20480
+    slots, 1100 keys): cut by the length for a single sequence too."""
+    import torch
+    rng = np.random.default_rng(80)
+    n, page, pages = 1100, 64, 320
+    cfg = cache_config(1, 1, page, pages, 1, 512, 0)
+    pt = fill_page_table(cfg, [n])
+    ck0 = np.full((pages * page, 1, 512), NAN)
+    cv0 = ck0.copy()
+    ck0[:n], cv0[:n] = randn_bf16(rng, (n, 1, 512)), randn_bf16(rng, (n, 1, 512))
+    q, k, v = (randn_bf16(rng, (1, h, 512)) for h in (16, 1, 1))
+    exp_k, exp_v = ck0.copy(), cv0.copy()
+    oracle.kv_cache_write(exp_k, exp_v, cfg, pt, [0], [n - 1], 0, k, v)
+    exp = oracle.decode_attention(q, exp_k, exp_v, pt, [n], cfg, 0, 0.0442)
+    c = gk.make_config(*cfg)
+    ws = torch.empty(gk.decode_step_workspace_bytes(1) // 4, dtype=torch.int32, device=dev)
+    gk.check(gk.decode_step_workspace_init(ws, 1))
+    ck, cv, out = to_dev(ck0, dev), to_dev(cv0, dev), to_dev(np.zeros_like(q), dev)
+    seq, pos = to_dev(np.int32([n]), dev), to_dev(np.int32([n - 1]), dev)
+    gk.check(gk.decode_step_layers_bf16(out, to_dev(q, dev), to_dev(k, dev), to_dev(v, dev), None, None, None, c,
+                                        ck, cv, to_dev(pt, dev), c, seq, pos, 5, 1, 0.0442, 1, ws))
+    torch.cuda.synchronize()
+    assert gk.decode_step_status(ws) == 0
+    assert np.array_equal(from_dev_bf16(ck).reshape(exp_k.shape), exp_k)
+    assert_close(from_dev_bf16(out), exp, "capacity plan")

@@ -1,0 +1,88 @@
+"""Global prefill chunks of few row blocks run their key tiles in parts on
+several workgroups, merged by a second launch through the workspace: the
+edges of row blocks, tiles and parts, ragged batches, smaller workspaces, and
+a balanced chunk on the same workspace afterwards."""
+import math
+
+import numpy as np
+import pytest
+
+import gemma_kv as gk
+from kvtest import assert_close, cache_config, empty_bf16, fill_page_table, from_dev_bf16, randn_bf16, to_dev
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+H, D = 8, 256
+SLOT_BYTES = 256 + 2 * 130 * 256 * 4
+
+
+def _run(dev, priors, lq, page, ws=None, ws_bytes=None, capacity=0):
+    import torch
+    rng = np.random.default_rng(lq * 7 + sum(priors))
+    batch = len(priors)
+    max_pages = max(capacity, max(priors) + lq) // page + 1
+    cfg = cache_config(1, batch, page, max_pages, H, D, 0)
+    pt = fill_page_table(cfg, priors)
+    q = randn_bf16(rng, (batch, lq, 16, D))
+    k, v = randn_bf16(rng, (batch, lq, H, D)), randn_bf16(rng, (batch, lq, H, D))
+    ck, cv = (randn_bf16(rng, (batch * max_pages * page, H, D)) for _ in range(2))
+    c = gk.make_config(*cfg)
+    need = gk.flash_attention_prefill_chunk_workspace_bytes(batch, lq, c)
+    if ws is None:
+        ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    args = [to_dev(x, dev) for x in (q, k, v, ck, cv, pt, np.asarray(priors, np.int32))]
+    scale = 1 / math.sqrt(D)
+    out, plain = empty_bf16((batch, lq, 16, D), dev), empty_bf16((batch, lq, 16, D), dev)
+    print(f"priors {priors} rows {lq} page {page} workspace {ws_bytes or ws.numel()}", flush=True)
+    gk.check(gk.flash_attention_prefill_chunk_paged_bf16_ws(
+        out, *args, c, 0, batch, lq, scale, ws, ws_bytes or ws.numel()))
+    gk.check(gk.flash_attention_prefill_chunk_paged_bf16(plain, *args, c, 0, batch, lq, scale))
+    torch.cuda.synchronize()
+    got = from_dev_bf16(out)
+    assert_close(got, from_dev_bf16(plain), f"parts vs plain {priors} {lq}")
+    rows = pt.reshape(batch, max_pages).astype(np.int64)
+    b = batch - 1
+    pos = np.arange(priors[b])
+    r = rows[b, pos // page] * page + pos % page
+    full = [np.concatenate([c0[r], new[b]])[None] for c0, new in ((ck, k), (cv, v))]
+    exp = oracle.prefill_attention(q[b:b + 1], *full, lq, priors[b] + lq, 16, H, D, 0, scale)[0]
+    assert_close(got[b], exp, f"parts vs oracle {priors} {lq}")
+    return ws
+
+
+@pytest.mark.parametrize("priors,lq,page", [
+    ([500], 1, 16),            # one row, one row block: 32 parts of two tiles at most
+    ([0], 64, 16),             # a single part: the chunk kernel writes the rows
+    ([128 - 64], 64, 16),      # two tiles, one part
+    ([129 - 64], 64, 64),      # three tiles: parts of two and one
+    ([900], 63, 1),
+    ([700], 65, 16),           # the second row block holds one row
+    ([3, 1200, 400], 17, 16),  # ragged: one, several and many parts
+    ([100], 400, 16),          # parts of the chunk's own keys
+    ([37], 1000, 16),          # two parts per row block
+])
+def test_parts_match_oracle(dev, priors, lq, page):
+    _run(dev, priors, lq, page, capacity=512)
+
+
+def test_parts_and_balanced_chunks_share_a_workspace(dev):
+    ws = _run(dev, [600], 40, 16)
+    ws = _run(dev, [9], 1100, 16, ws)    # 18 row blocks: balanced
+    ws = _run(dev, [600], 40, 16, ws)
+    assert not ws[: ws.numel() // SLOT_BYTES * SLOT_BYTES].view(-1, SLOT_BYTES)[:, :4].any().item()
+
+
+@pytest.mark.parametrize("slots", [0, 3, 8, 20])
+def test_smaller_workspaces_stay_accepted(dev, slots):
+    """A single row block needs no workspace; what there is gives fewer parts."""
+    import torch
+    ws = torch.zeros(max(slots, 1) * SLOT_BYTES, dtype=torch.uint8, device=dev)
+    _run(dev, [700], 50, 16, ws, max(1, slots * SLOT_BYTES))
+
+
+def test_workspace_bytes_never_shrink_with_the_call():
+    c = gk.make_config(*cache_config(1, 4, 64, 64, H, D, 0))
+    largest = gk.flash_attention_prefill_chunk_workspace_bytes(4, 2048, c)
+    for n in (1, 64, 65, 512, 1024, 1025, 2048):
+        sizes = [gk.flash_attention_prefill_chunk_workspace_bytes(b, n, c) for b in (1, 2, 4)]
+        assert sizes == sorted(sizes) and sizes[-1] <= largest
