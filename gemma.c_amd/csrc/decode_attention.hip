@@ -809,9 +809,12 @@ hipError_t launch_combine(const DecodeParams &p, int32_t batch_count, hipStream_
   };
   constexpr int kDims = combine_dims<kDim>();
   if constexpr (kDim == 512) {
-    if (p.balanced != 0 && batch_count > 4)
-      return launch(decode_combine_kernel<kDim, true, 4 * kDims>, 4 * kDims);
-    if (p.balanced != 0) return launch(decode_combine_kernel<kDim, true, kDims>, kDims);
+    const bool wide = batch_count > 4;
+    if (p.balanced != 0) {
+      return wide ? launch(decode_combine_kernel<kDim, true, 4 * kDims>, 4 * kDims)
+                  : launch(decode_combine_kernel<kDim, true, kDims>, kDims);
+    }
+    if (wide) return launch(decode_combine_kernel<kDim, false, 4 * kDims>, 4 * kDims);
   }
   return launch(decode_combine_kernel<kDim, false, kDims>, kDims);
 }
@@ -868,11 +871,13 @@ hipError_t decode_entry(uint16_t *out, float *pm, float *pl, float *pacc,
   // decode_geometry_ok: 8 x 256 or 1 x 512.
   const bool d512 = c.head_dim == 512;
   // A batch whose combine follows is cut by its lengths (balanced_cut): two
-  // workgroups per CU, all resident at once. One sequence is planned by its
+  // workgroups per CU, all resident at once. Not one that takes a single
+  // round of one-step workgroups as planned (2 x 500-1000 keys: 12.4 against 17 us). One sequence is planned by its
   // length already, except in a step (gate), which plans by the cache's
   // capacity: a cut there once that gives splits of more than one step.
+  const bool one_round = split_size <= kD512OneStep && (int64_t)num_splits * batch_count <= kD512Cus;
   if (d512 && combine && p.counters == nullptr && num_splits > 1 && batch_count <= kBalancedBatch &&
-      (batch_count >= 2 || (gate != nullptr && split_size > 4 * kD512TileKeys))) {
+      (batch_count >= 2 ? !one_round : (gate != nullptr && split_size > kD512OneStep))) {
     p.balanced = (int32_t)std::min((int64_t)num_splits * batch_count, (int64_t)kD512Workgroups);
     p.batch = batch_count;
   }
@@ -1087,8 +1092,7 @@ hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
     tile = SlidingShape::KT * SlidingShape::CT;  // one wave's page-lookup chunk
     key_tile = SlidingShape::KT;
   } else if (config.num_heads == 1 && config.head_dim == 512) {
-    tile = kD512TileKeys;
-    key_tile = kD512TileKeys / 2;
+    tile = key_tile = kD512TileKeys;
   } else {
     return hipErrorInvalidValue;
   }
@@ -1107,15 +1111,26 @@ hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
   int64_t size = (keys + splits_per_seq - 1) / splits_per_seq;
   size = ((size + tile - 1) / tile) * tile;
   if (size < tile) size = tile;
-  // Shorter splits of a 1 x 512 batch pay more for their start than they
-  // spread the work; the launch lengthens them to fit the chip (balanced_cut).
-  if (planned && config.head_dim == 512 && batch_count > 1) size = std::max<int64_t>(size, kD512BatchSplit);
+  // 1 x 512: a workgroup is one step of four 16-key waves or more, and starts
+  // slowly; 48 keys at least (4000 keys in splits of 16 / 32 / 48 / 64: 15.9 /
+  // 13.0 / 12.6 / 12.4 us). A batch takes single steps where they fit one
+  // round of the chip (8 of 100-1000 keys 12 us, 31 in splits of 16 on the
+  // former kernel), and kD512BatchSplit keys at least otherwise: the launch
+  // then sizes them by the lengths (balanced_cut).
+  if (planned && config.head_dim == 512) {
+    const int64_t steps = (keys + kD512OneStep - 1) / kD512OneStep;
+    if (steps == 1 || (batch_count > 1 && steps * batch_count <= kD512Cus)) {
+      size = kD512OneStep;
+    } else {
+      size = std::max<int64_t>(size, batch_count > 1 ? kD512BatchSplit : kD512OneStep - tile);
+    }
+  }
   // One sequence whose splits come out at two tiles or fewer (a sliding
   // layer's 1024-key window): the split is a dependent chain of tile
   // latencies, so one tile per workgroup, as long as that stays within two
   // workgroups per CU (1024 keys: 8.5 against 9.4 us per layer with the
   // combine, 512 against 256 workgroups).
-  if (planned && batch_count == 1 && size <= 2 * key_tile &&
+  if (planned && config.head_dim == 256 && batch_count == 1 && size <= 2 * key_tile &&
       heads * ((keys + key_tile - 1) / key_tile) <= 2 * target_workgroups) {
     size = key_tile;
   }

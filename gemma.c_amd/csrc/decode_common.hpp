@@ -211,6 +211,8 @@ bool decode_geometry_ok(const Gemma4KvCacheConfig &c, int32_t layer, int32_t bat
 
 // 1 x 512 split kernel (decode_d512.hip).
 constexpr int kD512TileKeys = 16;     // keys of a wave's tile
+constexpr int kD512OneStep = 64;      // longest split of the one-step, four-wave form
+constexpr int kD512Cus = 256;
 constexpr int kD512Workgroups = 512;  // balanced: two 69 KiB workgroups on each of 256 CUs
 // The plan's shortest split of a batch. 64 / 96 / 128 keys: 2 x 8193 20.9 / 18.9 /
 // 20.4 us, 8 x 100-4000 20.4 / 18.7 / 19.6 us, 16 x 30-1200 16.7 / 17.9 / 19.2 us.

@@ -668,7 +668,7 @@ hipError_t launch(const DecodeParams &p, int32_t batch_count, hipStream_t stream
 }  // namespace
 
 hipError_t launch_split_d512(const DecodeParams &p, int32_t batch_count, hipStream_t stream) {
-  return p.balanced == 0 && p.split_size <= 4 * kTileKeys ? launch<4>(p, batch_count, stream)
+  return p.balanced == 0 && p.split_size <= kD512OneStep ? launch<4>(p, batch_count, stream)
                                                           : launch<2>(p, batch_count, stream);
 }
 
