@@ -70,18 +70,6 @@ constexpr int kDimBlocks = kDim / 16;                   // blocks of O^T
 constexpr int kChunkTiles = kWave / kTileKeys;          // tiles per page lookup
 constexpr int kRot = kDim / 4;                          // rotary dims of a global head
 
-// Waits until at most n vector memory operations are outstanding, the
-// copies included.
-template <int n>
-__device__ __forceinline__ void wait_vector() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(n) : "memory");
-}
-// Waits for this wave's LDS reads: a copy issued next may overwrite what
-// they read.
-__device__ __forceinline__ void wait_lds_reads() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-}
-
 // Four whole rows (1 KiB each) into four consecutive LDS rows: 16 bytes per
 // lane from base[i] + off[i]. Few scalar instructions per row matter here (a
 // wave issues 32 rows before its first wait): M0 is saved once and stepped.

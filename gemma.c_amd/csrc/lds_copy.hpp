@@ -45,6 +45,39 @@ __device__ __forceinline__ void copy_dwords(const void *src, uint32_t lds_addr) 
       : [lds] "s"(lds_addr), [src] "v"(src));
 }
 
+// Two 1 KiB copies into consecutive LDS rows: 16 bytes per lane from
+// base + off0, then base + off1. base must not come straight from a vector
+// instruction (v_readlane: five wait states before a memory instruction reads
+// the SGPR, which the compiler does not see for inline asm).
+__device__ __forceinline__ void copy_lanes2(uint64_t base, uint32_t off0, uint32_t off1,
+                                            uint32_t lds_addr) {
+  uint32_t m0_saved;
+  asm volatile(
+      "s_mov_b32 %[m0s], m0\n\t"
+      "s_mov_b32 m0, %[lds]\n\t"
+      "s_nop 0\n\t"  // SALU write of M0 -> LDS DMA reading it: one wait state (gfx9)
+      "global_load_lds_dwordx4 %[o0], %[base]\n\t"
+      "s_add_u32 m0, m0, 1024\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %[o1], %[base]\n\t"
+      "s_mov_b32 m0, %[m0s]"
+      : [m0s] "=&s"(m0_saved)
+      : [lds] "s"(lds_addr), [base] "s"(base), [o0] "v"(off0), [o1] "v"(off1)
+      : "memory", "scc");
+}
+
+// Waits until at most n vector memory operations of this wave are
+// outstanding, the copies included.
+template <int n>
+__device__ __forceinline__ void wait_vector() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(n) : "memory");
+}
+// Waits for this wave's LDS reads: a copy issued next may overwrite what
+// they read.
+__device__ __forceinline__ void wait_lds_reads() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
 // Waits for every vector memory operation of this wave, the copies
 // included (s_waitcnt vmcnt(0); a builtin rather than inline asm so the
 // compiler's own counter bookkeeping sees it as well).

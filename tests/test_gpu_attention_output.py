@@ -106,3 +106,25 @@ def test_o_projection_argument_checks(dev):
     assert gk.attention_o_projection_post_norm_bf16(o, o, o, a, w, g, o, -1, 4096) != ok
     assert gk.attention_o_projection_post_norm_bf16(None, o, o, a, w, g, o, 1, 4096) != ok
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows,width", [
+    (2, 4096), (2, 8192), (16, 4096), (32, 8192), (33, 4096), (64, 8192), (65, 4096), (96, 4096),
+    (97, 4096), (128, 4096), (129, 4096), (192, 4096), (193, 4096), (256, 4096), (257, 4096), (131, 8192)])
+def test_o_projection_block_edges(dev, rows, width):
+    """Every split into row and column blocks at its edges, against the fp64
+    product (an fp32 sum of `width` products, then one bf16 rounding)."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows * 7 + width)
+    a = torch.randn((rows, width), generator=gen, device=dev).bfloat16()
+    w = torch.randn((HIDDEN, width), generator=gen, device=dev).bfloat16()
+    g = torch.ones(HIDDEN, device=dev).bfloat16()
+    x = torch.zeros((rows, HIDDEN), device=dev).bfloat16()
+    outs = [torch.full((rows, HIDDEN), float("nan"), device=dev).bfloat16() for _ in range(3)]
+    gk.check(gk.attention_o_projection_post_norm_bf16(*outs, a, w, g, x, rows, width))
+    exact = a.double() @ w.double().T
+    bound = exact.abs() * 2.0 ** -8 + (a.double().abs() @ w.double().abs().T) * 2.0 ** -24 * 16
+    assert bool(((outs[0].double() - exact).abs() <= bound).all())
+    scale = outs[0].double().square().mean(-1, keepdim=True).add(1e-6).rsqrt()
+    assert torch.allclose(outs[1].double(), outs[0].double() * scale, rtol=2.0 ** -7, atol=1e-6)
+    assert torch.equal(outs[2], outs[1])
