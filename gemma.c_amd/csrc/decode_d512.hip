@@ -28,10 +28,10 @@
 //                  LDS took 3.6 us of a 12 us launch (8193 keys in splits of
 //                  48).
 // Measured (MI355X), before (v_dot2 kernel) and now: one sequence of 8193 keys
-// in 171 splits of 48, launch 19.1 -> 9.4 us (in the kernel 7.2: 0.8 to the
-// first words, 2 until K and V have arrived at ~8 TB/s, 1 for q's
-// preparation, 1.5 scores to P.V, 1 for the partial stores); 24 sequences of
-// 200-12001 keys, 302 MB, 199 -> 65 us.
+// in 171 splits of 48, launch 19.1 -> 8.7 us (in the kernel 6.2: 0.8 to the
+// first words, 2.4 until K has arrived and q is prepared, 1.3 scores to P.V,
+// 1 for the partial stores; with V requested before q's preparation instead
+// of after it, 7.2); 24 sequences of 200-12001 keys, 302 MB, 199 -> 64 us.
 // Waves and splits: a split of up to 64 keys is one step of four waves. Longer
 // ones run on two waves in 69 KiB of LDS, so that a CU holds two workgroups
 // and one streams while the other starts, scores or stores (24 sequences in
@@ -363,15 +363,11 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   if (live0) {
 #pragma unroll
     for (int i = 0; i < kTileKeys; i += 4) copy_k4(0, i);
-    if constexpr (kOwnQ) {
-#pragma unroll
-      for (int i = 0; i < kTileKeys; i += 4) copy_v4(0, i);
-    }
   }
-  if (prep_token) {  // while the first tile is in flight
+  if (prep_token) {  // while the first K rows are in flight
     // cos and sin: everything before the tile's copies, if it has any.
     if (live0) {
-      wait_vector<(kOwnQ ? 2 : 1) * kTileKeys>();
+      wait_vector<kTileKeys>();
     } else {
       wait_vector<0>();
     }
@@ -397,6 +393,10 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   for (int i = 0; i < kWaveHeads; ++i) {
     const int head = wave * kWaveHeads + i;
     s_q[head * kRowChunks + (lane ^ head)] = q_row[i];
+  }
+  if (kOwnQ && live0) {
+#pragma unroll
+    for (int i = 0; i < kTileKeys; i += 4) copy_v4(0, i);
   }
   lds_barrier();
   uint4 q[kSteps];
