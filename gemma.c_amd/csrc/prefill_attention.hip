@@ -30,11 +30,15 @@
 //     rows x 32 bytes, which this layout spreads over all banks. The
 //     transposing read turns row-major V into the V^T operand directly.
 // Tile t+1 is copied while tile t is computed; one barrier per tile. The
-// copies are issued between block 1's score MFMAs (inline asm, so the
+// copies are issued between block 0's score MFMAs (inline asm, so the
 // compiler neither serialises them nor waits on them; each wave waits for
-// its own copies right before the barrier), the next tile's row addresses
-// are resolved between block 0's score MFMAs, and the page-table entries
-// those need arrive in LDS by a 4-byte copy issued two tiles ahead.
+// its own copies right before the barrier): as early as the stage is free, a
+// whole tile ahead of their use. Issued half a tile later, in block 1, their
+// latency showed wherever K and V came from HBM (2048 rows after 6144, three
+// sets of inputs in turn: 316 against 279 us). The row addresses of the tile
+// after the next are resolved between block 1's score MFMAs, and the
+// page-table entries those need arrive in LDS by a 4-byte copy issued a tile
+// before.
 // Each score block first issues all 16 of its K-fragment reads (into AGPRs),
 // then its MFMA chain, so LDS latency is paid once per block. The MFMAs use
 // the VGPR accumulator form (a build flag for this file): with AGPR
@@ -416,20 +420,18 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
     return (n ^ (((2 * a + half) & 3) << 2)) * 16;
   };
 
-  // Row addresses of the next tile: lane j < 16 resolves key 16w + j and
-  // publishes {K row, V row} in the wave's row table and the stage's validity
-  // bits; lane l then fetches key 16w + 2a + l/32 of copy a and adds its
+  // Row addresses of a tile: lane j < 16 resolves key 16w + j and publishes
+  // {K row, V row} in the wave's row table (the readable-key bits are
+  // returned: the tile's stage is still in use); lane l then fetches key 16w + 2a + l/32 of copy a and adds its
   // swizzled source chunk.
-  auto prepare_copy = [&](auto st, int kt, int32_t phys, uint64_t (&ksrc)[kCopyKeys / 2],
-                          uint64_t (&vsrc)[kCopyKeys / 2]) __attribute__((always_inline)) {
-    constexpr int S = decltype(st)::value;
+  auto prepare_copy = [&](int kt, int32_t phys, uint64_t (&ksrc)[kCopyKeys / 2],
+                          uint64_t (&vsrc)[kCopyKeys / 2]) __attribute__((always_inline)) -> uint32_t {
     uint4 rows;
     const bool ok = resolve(kt, phys, rows);
     const uint32_t ok_bits = (uint32_t)__builtin_amdgcn_ballot_w64(ok) & 0xFFFFu;
     // Lanes with equal lane % 16 hold equal rows, so every lane stores
     // (no divergent branch in the way of instruction scheduling).
     s_rows[wave][key_lane] = rows;
-    s_valid[S][wave] = ok_bits;
     uint4 rr[kCopyKeys / 2];
 #pragma unroll
     for (int a = 0; a < kCopyKeys / 2; ++a) rr[a] = s_rows[wave][2 * a + half];
@@ -438,6 +440,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
       ksrc[a] = (((uint64_t)rr[a].y << 32) | rr[a].x) + src_k(a);
       vsrc[a] = (((uint64_t)rr[a].w << 32) | rr[a].z) + src_v(a);
     }
+    return ok_bits;
   };
   // LDS byte address of this wave's copy destination in each stage.
   auto lds_addr = [](const void *ptr) __attribute__((always_inline)) -> uint32_t {
@@ -474,13 +477,15 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   for (int d = 0; d < DB; ++d) acc[d] = f32x16_t{};
 
   // One block of 32 keys: S^T, masked softmax, O^T += V^T P^T.
-  // Next-tile work rides on the two blocks of a tile: the row addresses
-  // are resolved (next_rows) while block 0's score MFMAs run, and the 16
-  // copies are issued between block 1's score MFMAs. Both happen even when
-  // a block itself is skipped.
+  // Later tiles' work rides on the two blocks of a tile: the 16 copies of
+  // the next tile are issued between block 0's score MFMAs, and the row
+  // addresses of the one after it are resolved (next_rows) while block 1's
+  // run. Both happen even when a block itself is skipped.
   uint64_t ksrc[kCopyKeys / 2], vsrc[kCopyKeys / 2];
+  uint32_t next_valid;  // readable keys of the prepared tile
   auto issue_copies = [&](auto st) __attribute__((always_inline)) {
     constexpr int S = decltype(st)::value;
+    s_valid[S ^ 1][wave] = next_valid;
 #pragma unroll
     for (int c = 0; c < kCopyKeys / 2; ++c) {
       copy_row_pair(ksrc[c], k_dst[S ^ 1] + c * 2 * kRowBytes);
@@ -488,17 +493,18 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
     }
   };
   auto attend_block = [&](auto st, auto blk, const char *vbase, int kb_lo, uint32_t valid32,
-                          bool copy, auto &&next_rows) __attribute__((always_inline)) {
+                          bool copy, bool needed, auto &&next_rows) __attribute__((always_inline)) {
     constexpr int S = decltype(st)::value;
     constexpr int kBlk = decltype(blk)::value;
     constexpr int kImm = S * kTileBytes + kBlk * 32 * kRowBytes;
     const int kb_hi = kb_lo + 31;
     if (!wave_has_rows || kb_lo > wave_qmax || (p.window > 0 && kb_hi <= wave_qmin - p.window)) {
-      if (copy) {
+      // Nothing to overlap with here: only what a later tile will use.
+      if (copy && needed) {
         if constexpr (kBlk == 0) {
-          next_rows();
-        } else {
           issue_copies(st);
+        } else {
+          next_rows();
         }
       }
       return;
@@ -517,7 +523,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
       s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[s]),
                                                       __builtin_bit_cast(bf16x8_t, qreg[s]), s_acc,
                                                       0, 0, 0);
-      if constexpr (kBlk == 1) {
+      if constexpr (kBlk == 0) {
         if (copy) {
           if constexpr (pos % 2 == 0) {
             copy_row_pair(ksrc[pos / 2], k_dst[S ^ 1] + (pos / 2) * 2 * kRowBytes);
@@ -530,8 +536,11 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    static_for<0, KS>(step_s);
     if constexpr (kBlk == 0) {
+      if (copy) s_valid[S ^ 1][wave] = next_valid;
+    }
+    static_for<0, KS>(step_s);
+    if constexpr (kBlk == 1) {
       if (copy) next_rows();
       // Interleave the address work with the score MFMAs.
       static_for<0, KS>([](auto) __attribute__((always_inline)) {
@@ -617,14 +626,20 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
     __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
   };
 
-  // ---- pipeline: copy tile i+1 and look up tile i+2 while computing i -----
+  // ---- pipeline: copy tile i+1 and resolve tile i+2 while computing i -----
   // The page-table entries of tile t land in s_pages[t & 1] by LDS copy,
-  // issued two tiles ahead, so no vector register waits on them.
+  // issued three tiles ahead, so no vector register waits on them.
   const uint32_t page_dst[2] = {(uint32_t)wave_uniform(lds_addr(&s_pages[0][wave][0])),
                                 (uint32_t)wave_uniform(lds_addr(&s_pages[1][wave][0]))};
-  prepare_copy(Stage<0>{}, tile0, *page_entry(tile0), ksrc, vsrc);
+  // Both entries before the first copy: the wait for the second would wait for
+  // the copies too (and then tile 1's addresses follow instead of overlapping).
+  const int32_t phys0 = *page_entry(tile0);
+  int32_t phys1 = *page_entry(tile0 + kTileKeys);
+  asm volatile("" : "+v"(phys1));
+  next_valid = prepare_copy(tile0, phys0, ksrc, vsrc);
   issue_copies(Stage<1>{});  // into stage 0
-  copy_dwords(page_entry(tile0 + kTileKeys), page_dst[1]);
+  copy_dwords(page_entry(tile0 + 2 * kTileKeys), page_dst[0]);
+  next_valid = prepare_copy(tile0 + kTileKeys, phys1, ksrc, vsrc);
   auto step = [&](auto st, int it) __attribute__((always_inline)) {
     constexpr int S = decltype(st)::value;
     const int kt = tile0 + it * kTileKeys;
@@ -633,20 +648,20 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
     wait_copies();
     __syncthreads();
     // The copy after the last tile reads keys past the workgroup's range,
-    // which resolve to the (always readable) first chunk row: the loop has
-    // no branches around its copies.
+    // which resolve to the (always readable) first chunk row, or repeats rows
+    // resolved before: a computed block has no branches around its copies.
     constexpr bool copy = true;
-    const int32_t next_phys = s_pages[S ^ 1][wave][lane];
+    const int32_t next_phys = s_pages[S][wave][lane];
     auto next_rows = [&]() __attribute__((always_inline)) {
-      prepare_copy(Stage<S ^ 1>{}, kt + kTileKeys, next_phys, ksrc, vsrc);
-      copy_dwords(page_entry(kt + 2 * kTileKeys), page_dst[S]);
+      next_valid = prepare_copy(kt + 2 * kTileKeys, next_phys, ksrc, vsrc);
+      copy_dwords(page_entry(kt + 3 * kTileKeys), page_dst[S ^ 1]);
     };
     const char *vbase = reinterpret_cast<const char *>(S == 0 ? s_v0 : s_v1);
     const uint4 vw = *reinterpret_cast<const uint4 *>(&s_valid[S][0]);
     attend_block(st, std::integral_constant<int, 0>{}, vbase, kt, vw.x | (vw.y << 16), copy,
-                 next_rows);
+                 it + 1 < n_tiles, next_rows);
     attend_block(st, std::integral_constant<int, 1>{}, vbase + 32 * kRowBytes, kt + 32,
-                 vw.z | (vw.w << 16), copy, next_rows);
+                 vw.z | (vw.w << 16), copy, it + 2 < n_tiles, next_rows);
   };
   for (int it = 0; it < n_tiles; it += 2) {
     step(Stage<0>{}, it);
