@@ -53,11 +53,11 @@ __device__ __forceinline__ void load_run(const uint16_t *src, float (&x)[kPer]) 
 template <int kPer>
 __device__ __forceinline__ void store_run(uint16_t *dst, const float (&y)[kPer]) {
   if constexpr (kPer == 4) {
-    *reinterpret_cast<uint2 *>(dst) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+    *reinterpret_cast<uint2 *>(dst) = make_uint2(cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3]));
   } else {
     *reinterpret_cast<uint4 *>(dst) =
-        make_uint4(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]), pack_bf16x2(y[4], y[5]),
-                   pack_bf16x2(y[6], y[7]));
+        make_uint4(cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3]), cvt_pk_bf16(y[4], y[5]),
+                   cvt_pk_bf16(y[6], y[7]));
   }
 }
 
