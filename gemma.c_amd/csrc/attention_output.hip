@@ -139,11 +139,12 @@ __global__ __launch_bounds__(kSplit *kWave) void o_projection_kernel(
     const uint64_t k = (uint64_t)chunk * kChunkK * 2;
 #pragma unroll
     for (int b = 0; b < kColBlocks; ++b)
-      copy_lanes2(w_base + k + (uint64_t)b * 16 * kWidth * 2, w_off[0], w_off[1],
-                  lds + b * kBlockUint4 * 16);
+      copy_lanes2(w_base + k + (uint64_t)b * 16 * kWidth * 2, w_off[0],
+                  w_base + k + (uint64_t)b * 16 * kWidth * 2, w_off[1], lds + b * kBlockUint4 * 16);
 #pragma unroll
     for (int b = 0; b < kRowBlocks; ++b)
-      copy_lanes2(a_base + k, a_off[b][0], a_off[b][1], lds + (kColBlocks + b) * kBlockUint4 * 16);
+      copy_lanes2(a_base + k, a_off[b][0], a_base + k, a_off[b][1],
+                  lds + (kColBlocks + b) * kBlockUint4 * 16);
   };
 
   // Few blocks leave registers for four sums each: shorter chains, a smaller

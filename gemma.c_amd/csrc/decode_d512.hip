@@ -107,12 +107,6 @@ __device__ __forceinline__ uint64_t lane_address(uint64_t v, int from) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// Workgroup barrier that orders LDS traffic only: the copies in flight stay
-// in flight (__syncthreads may wait for them).
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 template <int kWaves>
 __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(DecodeParams p) {
   constexpr int kWaveBlocks = kDimBlocks / kWaves;  // 16-dim blocks of O^T per wave

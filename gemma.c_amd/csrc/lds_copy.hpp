@@ -46,23 +46,23 @@ __device__ __forceinline__ void copy_dwords(const void *src, uint32_t lds_addr) 
 }
 
 // Two 1 KiB copies into consecutive LDS rows: 16 bytes per lane from
-// base + off0, then base + off1. base must not come straight from a vector
+// base0 + off0, then base1 + off1. The bases must not come straight from a vector
 // instruction (v_readlane: five wait states before a memory instruction reads
 // the SGPR, which the compiler does not see for inline asm).
-__device__ __forceinline__ void copy_lanes2(uint64_t base, uint32_t off0, uint32_t off1,
-                                            uint32_t lds_addr) {
+__device__ __forceinline__ void copy_lanes2(uint64_t base0, uint32_t off0, uint64_t base1,
+                                            uint32_t off1, uint32_t lds_addr) {
   uint32_t m0_saved;
   asm volatile(
       "s_mov_b32 %[m0s], m0\n\t"
       "s_mov_b32 m0, %[lds]\n\t"
       "s_nop 0\n\t"  // SALU write of M0 -> LDS DMA reading it: one wait state (gfx9)
-      "global_load_lds_dwordx4 %[o0], %[base]\n\t"
+      "global_load_lds_dwordx4 %[o0], %[b0]\n\t"
       "s_add_u32 m0, m0, 1024\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %[o1], %[base]\n\t"
+      "global_load_lds_dwordx4 %[o1], %[b1]\n\t"
       "s_mov_b32 m0, %[m0s]"
       : [m0s] "=&s"(m0_saved)
-      : [lds] "s"(lds_addr), [base] "s"(base), [o0] "v"(off0), [o1] "v"(off1)
+      : [lds] "s"(lds_addr), [b0] "s"(base0), [b1] "s"(base1), [o0] "v"(off0), [o1] "v"(off1)
       : "memory", "scc");
 }
 
@@ -76,6 +76,12 @@ __device__ __forceinline__ void wait_vector() {
 // they read.
 __device__ __forceinline__ void wait_lds_reads() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
+// Workgroup barrier that orders LDS traffic only: the copies in flight stay
+// in flight (__syncthreads may wait for them).
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // Waits for every vector memory operation of this wave, the copies

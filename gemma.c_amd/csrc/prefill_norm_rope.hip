@@ -11,7 +11,8 @@
 //      the 8x256 geometry reuses the chunk kernel (no prior context), the
 //      1x512 geometry runs prefill_d512_kernel below.
 //
-// prefill_d512_kernel: 16 query heads share one 512-dim KV head. A wave owns
+// prefill_d512_short_kernel (sequences up to kD512ShortRows): 16 query heads
+// share one 512-dim KV head. A wave owns
 // one query row and all 16 heads (16 MFMA columns) on
 // v_mfma_f32_16x16x32_bf16, computing S^T = K Q^T (16 keys x 16 heads per
 // block, 16 k-steps of 32 dims) and O^T = V^T P^T (32 dim blocks of 16). In
@@ -29,8 +30,18 @@
 // MFMA (one counter wait per MFMA, two accumulator chains), and the P.V
 // phase keeps its transposing V reads four MFMAs ahead. The lazy online
 // softmax of the chunk kernel (maximum moved only when it grows by more than
-// 8 in log2 units). Per 32-key tile a wave reads 64 KiB of K and V from LDS
-// for 16 query columns, so the kernel is bound by LDS reads, not MFMA.
+// 8 in log2 units).
+//
+// prefill_d512_kernel (longer ones): the same tiles and operands on two waves
+// per row. Each scores 16 of a tile's 32 keys and, for all four rows, weighs
+// V in its own 64 dims, so that one V operand serves four MFMAs (32 instead of
+// 128 KiB of V reads per tile and CU) and two waves per SIMD cover each
+// other's LDS latency; maxima and probabilities travel through LDS. Three
+// tiles are in work at once and one barrier separates iterations. What bounds
+// it: the sum of many short LDS round trips, ~4000 clocks per 32-key iteration
+// against 1024 of MFMA. 2048 / 1024 / 777 rows, prep included: 148.6 / 64.0 /
+// 54.7 us against 163.2 / 74.0 / 61.1 on the short form; without the
+// overlap of tiles 151.7 / 68.0 / 57.3. Back to back, 2048 rows: 155 -> 132.
 #include "gemma4_device.hpp"
 #include "lds_copy.hpp"
 #include "prep_common.hpp"
@@ -124,14 +135,20 @@ __global__ __launch_bounds__((prep_waves<kHeads, kHasV>() * kWave)) void prefill
 }
 
 // ---- 1x512 causal self-attention ---------------------------------------
+// Up to this many rows the short form is faster (100 rows 21.3 against 23.4 us:
+// the long form fills its pipeline of three tiles first; 333 rows 34.6 / 34.1).
+constexpr int kD512ShortRows = 256;
 constexpr int kD512 = 512;
-constexpr int kD512Rows = 4;          // query rows (one per wave) per workgroup
-constexpr int kD512Threads = kD512Rows * kWave;
+constexpr int kD512Rows = 4;          // query rows per workgroup, two waves each
+constexpr int kD512Waves = 2 * kD512Rows;
+constexpr int kD512Threads = kD512Waves * kWave;
+constexpr int kD512ShortThreads = kD512Rows * kWave;  // the short form: a wave per row
+constexpr int kD512VLead = 4;         // its P.V MFMAs the V reads run ahead
 constexpr int kD512Tile = 32;         // keys per LDS tile
 constexpr int kD512RowBytes = kD512 * 2;
 constexpr int kD512Chunks = kD512RowBytes / 16;  // 16-byte chunks per row
 constexpr float kD512Slack = 8.0f;
-constexpr int kD512VLead = 4;         // P.V MFMAs the V reads run ahead
+constexpr int kD512Blocks = kD512 / 16 / kD512Waves;  // 16-dim blocks of O^T per wave
 
 struct D512Params {
   uint16_t *out;        // [B][L][16][512]
@@ -157,7 +174,7 @@ typedef unsigned u32x4v_t __attribute__((ext_vector_type(4)));
 // is at (base ^ (64 (s & 3))) + 256 (s >> 2): four XORed addresses, four
 // immediate offsets each. Issue position p = 4 (s & 3) + (s >> 2).
 template <int kImm>
-__device__ __forceinline__ void d512_read_kfrags(uint32_t k_addr, u32x4v_t (&kf)[16]) {
+__device__ __forceinline__ void d512_read_block(uint32_t k_addr, u32x4v_t (&kf)[16]) {
   uint32_t t0, t1;
   asm volatile(
       "s_waitcnt lgkmcnt(0)\n\t"
@@ -189,11 +206,44 @@ __device__ __forceinline__ void d512_read_kfrags(uint32_t k_addr, u32x4v_t (&kf)
       : [ka] "v"(k_addr), [i0] "i"(kImm), [i1] "i"(kImm + 256), [i2] "i"(kImm + 512),
         [i3] "i"(kImm + 768));
 }
-// Issue position of k-step s in d512_read_kfrags.
-constexpr int d512FragPos(int s) { return 4 * (s & 3) + (s >> 2); }
+// Issue position of k-step s in d512_read_block.
+constexpr int d512BlockPos(int s) { return 4 * (s & 3) + (s >> 2); }
 template <int kStep>
+__device__ __forceinline__ void d512_block_ready(u32x4v_t &f) {
+  asm volatile("s_waitcnt lgkmcnt(%[n])" : "+a"(f) : [n] "i"(15 - d512BlockPos(kStep)));
+}
+// Half of the 16 K-fragment reads of one 16-key score block into AGPRs, all
+// eight in flight before their first MFMA. For lane key k (k & 15 = lane & 15)
+// and lane group g, k-step s sits at chunk (4s + g) ^ (k & 15) of the key's
+// row: bits 0-1 of the chunk are g ^ (k & 3), bits 2-3 are (s & 3) ^
+// ((k >> 2) & 3) and bits 4+ are s >> 2. So with base = the address of k-step
+// 0, k-step s is at (base ^ (64 (s & 3))) + 256 (s >> 2): two XORed addresses
+// per half, four immediate offsets each. Fragment i of half kHalf is k-step
+// 2 kHalf + i / 4 + 4 (i % 4).
+template <int kHalf>
+__device__ __forceinline__ void d512_read_kfrags(uint32_t k_addr, u32x4v_t (&kf)[8]) {
+  uint32_t t0, t1;
+  asm volatile(
+      "s_waitcnt lgkmcnt(0)\n\t"
+      "v_xor_b32 %[t0], %[x0], %[ka]\n\t"
+      "ds_read_b128 %[f0], %[t0] offset:%[i0]\n\t"
+      "ds_read_b128 %[f1], %[t0] offset:%[i1]\n\t"
+      "ds_read_b128 %[f2], %[t0] offset:%[i2]\n\t"
+      "ds_read_b128 %[f3], %[t0] offset:%[i3]\n\t"
+      "v_xor_b32 %[t1], %[x1], %[ka]\n\t"
+      "ds_read_b128 %[f4], %[t1] offset:%[i0]\n\t"
+      "ds_read_b128 %[f5], %[t1] offset:%[i1]\n\t"
+      "ds_read_b128 %[f6], %[t1] offset:%[i2]\n\t"
+      "ds_read_b128 %[f7], %[t1] offset:%[i3]"
+      : [t0] "=&v"(t0), [t1] "=&v"(t1), [f0] "=&a"(kf[0]), [f1] "=&a"(kf[1]), [f2] "=&a"(kf[2]),
+        [f3] "=&a"(kf[3]), [f4] "=&a"(kf[4]), [f5] "=&a"(kf[5]), [f6] "=&a"(kf[6]), [f7]
+        "=&a"(kf[7])
+      : [ka] "v"(k_addr), [x0] "i"(128 * kHalf), [x1] "i"(128 * kHalf + 64), [i0] "i"(0),
+        [i1] "i"(256), [i2] "i"(512), [i3] "i"(768));
+}
+template <int kPos>
 __device__ __forceinline__ void d512_kfrag_ready(u32x4v_t &f) {
-  asm volatile("s_waitcnt lgkmcnt(%[n])" : "+a"(f) : [n] "i"(15 - d512FragPos(kStep)));
+  asm volatile("s_waitcnt lgkmcnt(%[n])" : "+a"(f) : [n] "i"(7 - kPos));
 }
 template <int kBegin, int kEnd, class F>
 __device__ __forceinline__ void d512_static_for(F &&f) {
@@ -203,7 +253,262 @@ __device__ __forceinline__ void d512_static_for(F &&f) {
   }
 }
 
-__global__ __launch_bounds__(kD512Threads, 1) void prefill_d512_kernel(D512Params p) {
+__global__ __launch_bounds__(kD512Threads) void prefill_d512_kernel(D512Params p) {
+  constexpr int KS = kD512 / 32;  // 32-dim k-steps of S^T
+  // Two stages of K and V tiles (32 keys x 1 KiB each), and what the waves
+  // trade, by the parity of the tile: each row's maxima over a wave's 16 keys,
+  // the probabilities as B operands (one wave's keys in each half), the
+  // rescale of the row's accumulators where its maximum moved; at the end the
+  // rows' sums.
+  struct Lds {
+    uint4 k[2][kD512Tile * kD512Chunks];
+    uint4 v[2][kD512Tile * kD512Chunks];
+    uint2 p[2][kD512Rows][kWave][2];
+    float max[2][kD512Rows][2][kQueryHeads];
+    float alpha[2][kD512Rows][kQueryHeads];
+    int32_t moved[2][kD512Rows];
+    float sum[kD512Rows][2][kQueryHeads];
+  };
+  __shared__ __attribute__((aligned(1024))) Lds lds;
+
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = wave_uniform(t >> 6);
+  const int my_row = wave >> 1;  // row of the workgroup
+  const int blk = wave & 1;      // its 16 keys of every tile
+  const int head = lane & 15;    // MFMA column
+  const int g = lane >> 4;       // lane group: keys / dims 4g..4g+3 of the accumulator
+  const int b = blockIdx.y;
+  const int L = p.seq_len;
+  // Causal work grows with the row: the last rows are dispatched first, so
+  // the workgroups of the first rows fill the CUs that free up early
+  // (longest-first order; one workgroup per CU at a time).
+  const int r0 = (gridDim.x - 1 - blockIdx.x) * kD512Rows;
+  const int row = r0 + my_row;
+  const int last_key = min(r0 + kD512Rows, L) - 1;  // last key any row of the workgroup sees
+
+  // Q^T operand: lane holds Q[row][head][32 s + 8 g .. +8] for k-step s. A row
+  // past the sequence computes the last one's scores and is not stored.
+  uint4 qreg[KS];
+  {
+    const uint16_t *qrow =
+        p.q + (((int64_t)b * L + min(row, L - 1)) * kQueryHeads + head) * kD512 + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qreg[s] = load128(qrow + 32 * s);
+    // Q lives in AGPRs (an MFMA operand may be an AGPR); all loads are
+    // issued before the first constraint forces a wait.
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      u32x4v_t t4 = {qreg[s].x, qreg[s].y, qreg[s].z, qreg[s].w};
+      asm volatile("" : "+a"(t4));
+      qreg[s] = make_uint4(t4.x, t4.y, t4.z, t4.w);
+    }
+  }
+
+  float m_run = -INFINITY, l_run = 0.0f;  // of this wave's row
+  f32x4_t acc[kD512Rows][kD512Blocks];    // every row's, this wave's dims
+#pragma unroll
+  for (int r = 0; r < kD512Rows; ++r)
+#pragma unroll
+    for (int d = 0; d < kD512Blocks; ++d) acc[r][d] = f32x4_t{};
+
+  const uint64_t kseq = reinterpret_cast<uint64_t>(p.k + (int64_t)b * L * kD512);
+  const uint64_t vseq = reinterpret_cast<uint64_t>(p.v + (int64_t)b * L * kD512);
+  const int n_tiles = last_key / kD512Tile + 1;
+  // Copy of a tile into a stage: wave w copies keys 4w .. 4w+3, one 1 KiB row
+  // per copy; lane l fills LDS chunk l with the swizzled source chunk. Past
+  // the sequence's end its last row is repeated (and masked). All but one XOR
+  // per row is scalar: the registers are full.
+  constexpr int kCopyRows = kD512Tile / kD512Waves;
+  constexpr int kPairs = kCopyRows / 2;
+  constexpr int kStageBytes = kD512Tile * kD512RowBytes;
+  const uint32_t lane_bytes = lane * 16;
+  const uint32_t k_dst = wave_uniform(lds_address(&lds.k[0][kCopyRows * wave * kD512Chunks]));
+  const uint32_t v_dst = wave_uniform(lds_address(&lds.v[0][kCopyRows * wave * kD512Chunks]));
+  auto row_base = [&](uint64_t seq, int kt, int key) __attribute__((always_inline)) {
+    return seq + (uint64_t)(uint32_t)min(kt + key, L - 1) * kD512RowBytes;
+  };
+  auto copy_k = [&](int kt, int stage, int i) __attribute__((always_inline)) {
+    const int key = kCopyRows * wave + 2 * i;
+    copy_lanes2(row_base(kseq, kt, key), lane_bytes ^ (16 * (key & 15)),
+                row_base(kseq, kt, key + 1), lane_bytes ^ (16 * ((key + 1) & 15)),
+                k_dst + stage * kStageBytes + i * 2 * kD512RowBytes);
+  };
+  auto copy_v = [&](int kt, int stage, int i) __attribute__((always_inline)) {
+    const int key = kCopyRows * wave + 2 * i;
+    copy_lanes2(row_base(vseq, kt, key), lane_bytes ^ (32 * (key & 7)),
+                row_base(vseq, kt, key + 1), lane_bytes ^ (32 * ((key + 1) & 7)),
+                v_dst + stage * kStageBytes + i * 2 * kD512RowBytes);
+  };
+  const int k15 = lane & 15;
+  const uint32_t k_base = lds_address(&lds.k[0][0]) + (16 * blk + k15) * kD512RowBytes +
+                          16 * (g ^ (k15 & 3)) + 64 * ((k15 >> 2) & 3);
+  // V^T operand of dim block d: lane i of group g reads rows k0 + j,
+  // dims 16 d + 4 q (j = (lane % 16) / 4, q = lane % 4) with k0 = 4 g and
+  // 16 + 4 g; chunk 2 (4 wave + d) + q / 2 of a row at c ^ 2 (row % 8).
+  const int vj = (lane & 15) >> 2, vq = lane & 3;
+  const int v_row = 4 * g + vj;  // and 16 + 4 g + vj, the same modulo 8
+  const int v_lane = v_row * kD512RowBytes + (wave >> 1) * 256 + ((vq >> 1) << 4) + ((vq & 1) << 3);
+
+  // Three tiles are in work at once, so that an iteration needs one barrier
+  // and its parts do not wait for each other: scores of tile it, softmax of
+  // tile it - 1 (whose maxima the barrier made known to both waves of a row),
+  // P.V of tile it - 2. Tiles -1 and -2 have probability 0 and meet zeroed V
+  // stages; past the last tile every key is masked.
+#pragma unroll
+  for (int i = 0; i < kPairs; ++i) copy_k(0, 0, i);
+  for (int i = t; i < 2 * kD512Tile * kD512Chunks; i += kD512Threads)
+    lds.v[0][i] = make_uint4(0, 0, 0, 0);
+  lds.p[0][my_row][lane][blk] = make_uint2(0, 0);
+  if (lane < kQueryHeads) lds.max[1][my_row][blk][lane] = -INFINITY;
+  if (lane == 0) lds.moved[0][my_row] = 0;
+  float sc[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};  // of tile it - 1
+
+#pragma unroll 1
+  for (int it = 0; it < n_tiles + 2; ++it) {
+    const int S = it & 1;  // parity of tiles it and it - 2
+    // Each wave waits for its own copies, the barrier for all: K of tile it,
+    // V of tile it - 2; and every wave is done with iteration it - 1.
+    wait_copies();
+    lds_barrier();
+    const float other_max = lds.max[S ^ 1][my_row][blk ^ 1][head];
+    const float own_max = lds.max[S ^ 1][my_row][blk][head];
+    int32_t moved[kD512Rows];
+    uint4 pb[kD512Rows];
+#pragma unroll
+    for (int r = 0; r < kD512Rows; ++r) {
+      moved[r] = lds.moved[S][r];
+      pb[r] = *reinterpret_cast<const uint4 *>(&lds.p[S][r][lane][0]);
+    }
+    auto v_operand = [&](int d) __attribute__((always_inline)) {
+      uint2 half_op[2];
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const char *addr = reinterpret_cast<const char *>(lds.v[S]) + v_lane +
+                           16 * r * kD512RowBytes +
+                           (((kD512Blocks * (wave & 1) + d) ^ (v_row & 7)) << 5);
+        typedef __attribute__((address_space(3))) i16x4_t lds_i16x4;
+        const i16x4_t tr = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_i16x4 *)(__attribute__((address_space(3))) const char *)(addr));
+        half_op[r] = __builtin_bit_cast(uint2, tr);
+      }
+      return make_uint4(half_op[0].x, half_op[0].y, half_op[1].x, half_op[1].y);
+    };
+    // P.V of tile it - 2, in two halves around the scores (their operands do
+    // not fit the registers together); one V operand serves the four rows.
+    uint4 vt[2] = {v_operand(0), v_operand(1)};
+#pragma unroll
+    for (int r = 0; r < kD512Rows; ++r) {
+      if (wave_uniform(moved[r]) == 0) continue;
+      const float alpha = lds.alpha[S][r][head];
+#pragma unroll
+      for (int d = 0; d < kD512Blocks; ++d) acc[r][d] *= alpha;
+    }
+    // Scores of tile it, half of the k-steps at a time: the fragments arrive
+    // under the P.V and the softmax. The copies of K of tile it + 1 and V of
+    // tile it - 1 ride on the MFMAs (the last K tile is copied again, unread:
+    // no branch around those).
+    const int kt = it * kD512Tile;
+    const int next_k = min(it + 1, n_tiles - 1) * kD512Tile;
+    const int next_v = min(it - 1, n_tiles - 1) * kD512Tile;
+    f32x4_t s2[2] = {f32x4_t{}, f32x4_t{}};
+    auto score_half = [&](auto hc, u32x4v_t (&kf)[8]) __attribute__((always_inline)) {
+      constexpr int kHalf = decltype(hc)::value;
+      d512_static_for<0, 8>([&](auto pc) __attribute__((always_inline)) {
+        constexpr int pos = decltype(pc)::value;
+        constexpr int s = 2 * kHalf + pos / 4 + 4 * (pos % 4);
+        d512_kfrag_ready<pos>(kf[pos]);
+        s2[pos & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8_t, kf[pos]), __builtin_bit_cast(bf16x8_t, qreg[s]),
+            s2[pos & 1], 0, 0, 0);
+        if constexpr (kHalf == 0 && pos % 4 == 1) {
+          if (next_v >= 0) copy_v(next_v, S ^ 1, pos / 4);
+        }
+        if constexpr (kHalf == 1 && pos % 4 == 1) copy_k(next_k, S ^ 1, pos / 4);
+        // Keep each fragment's wait right before its MFMA: without this
+        // fence the scheduler issued all the waits first, one lgkmcnt(0) in
+        // effect, and the reads no longer overlapped the MFMAs.
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    u32x4v_t kf[8];
+    d512_read_kfrags<0>(k_base + S * kStageBytes, kf);
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int r = 0; r < kD512Rows; ++r) acc[r][d] = mfma16(vt[d], pb[r], acc[r][d]);
+
+    score_half(std::integral_constant<int, 0>{}, kf);
+    d512_read_kfrags<1>(k_base + S * kStageBytes, kf);
+
+    // Softmax of tile it - 1.
+    const float tmax = fmaxf(own_max, other_max) * p.q_scale;
+    const bool moves = __builtin_amdgcn_ballot_w64(tmax > m_run + kD512Slack) != 0;
+    if (moves) {
+      const float m_new = fmaxf(m_run, tmax);
+      const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= alpha;
+      m_run = m_new;
+      if (lane < kQueryHeads) lds.alpha[S ^ 1][my_row][lane] = alpha;  // the same from both waves
+    }
+    const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+    float pr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      pr[j] = __builtin_amdgcn_exp2f(fmaf(sc[j], p.q_scale, -m_use));
+      l_run += pr[j];
+    }
+    lds.p[S ^ 1][my_row][lane][blk] =
+        make_uint2(cvt_pk_bf16(pr[0], pr[1]), cvt_pk_bf16(pr[2], pr[3]));
+    if (lane == 0) lds.moved[S ^ 1][my_row] = moves ? 1 : 0;
+
+    score_half(std::integral_constant<int, 1>{}, kf);
+    // Lane holds head `head`, keys 16 blk + 4 g + i.
+#pragma unroll
+    for (int d = 0; d < 2; ++d) vt[d] = v_operand(2 + d);
+    const f32x4_t score = s2[0] + s2[1];
+    float smax = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sc[j] = kt + 16 * blk + 4 * g + j <= row ? score[j] : -INFINITY;
+      smax = fmaxf(smax, sc[j]);
+    }
+    smax = xor_max<16>(smax);
+    smax = xor_max<32>(smax);
+    if (lane < kQueryHeads) lds.max[S][my_row][blk][lane] = smax;
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int r = 0; r < kD512Rows; ++r) acc[r][2 + d] = mfma16(vt[d], pb[r], acc[r][2 + d]);
+  }
+  static_assert(kPairs == 2, "two pairs of copies per operand");
+
+  wait_copies();  // no copy may still be writing LDS when the workgroup exits
+
+  // Normalise and store: lane holds head `head`, dims
+  // 16 (wave * kD512Blocks + d) + 4 g + i of every row.
+  l_run = xor_sum<16>(l_run);
+  l_run = xor_sum<32>(l_run);
+  if (lane < kQueryHeads) lds.sum[my_row][blk][lane] = l_run;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kD512Rows; ++r) {
+    if (r0 + r >= L) break;
+    const float sum = lds.sum[r][0][head] + lds.sum[r][1][head];
+    const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+    uint16_t *orow = p.out + (((int64_t)b * L + r0 + r) * kQueryHeads + head) * kD512 +
+                     wave * kD512Blocks * 16 + 4 * g;
+#pragma unroll
+    for (int d = 0; d < kD512Blocks; ++d) {
+      const f32x4_t o = acc[r][d] * inv;
+      *reinterpret_cast<uint2 *>(orow + 16 * d) =
+          make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+    }
+  }
+}
+
+// The short form: one wave per row, no exchange between waves.
+__global__ __launch_bounds__(kD512ShortThreads, 1) void prefill_d512_short_kernel(D512Params p) {
   constexpr int KS = kD512 / 32;  // 32-dim k-steps of S^T
   constexpr int DB = kD512 / 16;  // 16-dim blocks of O^T
   // Two stages of K and V tiles (32 keys x 1 KiB each).
@@ -255,7 +560,7 @@ __global__ __launch_bounds__(kD512Threads, 1) void prefill_d512_kernel(D512Param
   const int n_tiles = last_key / kD512Tile + 1;
   // Copy of a tile into a stage: wave w copies keys 8w .. 8w+7, one 1 KiB
   // row per copy; lane l fills LDS chunk l with the swizzled source chunk.
-  constexpr int kCopyRows = kD512Tile / (kD512Threads / kWave);
+  constexpr int kCopyRows = kD512Tile / (kD512ShortThreads / kWave);
   auto copy_tile = [&](int kt, int stage) {
 #pragma unroll
     for (int i = 0; i < kCopyRows; ++i) {
@@ -292,12 +597,12 @@ __global__ __launch_bounds__(kD512Threads, 1) void prefill_d512_kernel(D512Param
       constexpr int kImm =
           decltype(st)::value * kStageBytes + decltype(bl)::value * 16 * kD512RowBytes;
       u32x4v_t kf[16];
-      d512_read_kfrags<kImm>(k_base, kf);
+      d512_read_block<kImm>(k_base, kf);
       f32x4_t s2[2] = {f32x4_t{}, f32x4_t{}};
       d512_static_for<0, 16>([&](auto pc) __attribute__((always_inline)) {
         constexpr int pos = decltype(pc)::value;
         constexpr int s = 4 * (pos & 3) + (pos >> 2);  // k-step at issue position pos
-        d512_kfrag_ready<s>(kf[s]);
+        d512_block_ready<s>(kf[s]);
         s2[pos & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             __builtin_bit_cast(bf16x8_t, kf[s]), __builtin_bit_cast(bf16x8_t, qreg[s]),
             s2[pos & 1], 0, 0, 0);
@@ -342,7 +647,7 @@ __global__ __launch_bounds__(kD512Threads, 1) void prefill_d512_kernel(D512Param
       const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[j], p.q_scale, -m_use));
       const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[j + 1], p.q_scale, -m_use));
       l_run += p0 + p1;
-      pw[j / 2] = pack_bf16x2(p0, p1);
+      pw[j / 2] = cvt_pk_bf16(p0, p1);
     }
     const uint4 pb = make_uint4(pw[0], pw[1], pw[2], pw[3]);
     // V^T operand of dim block d: lane i of group g reads rows k0 + j,
@@ -395,6 +700,9 @@ __global__ __launch_bounds__(kD512Threads, 1) void prefill_d512_kernel(D512Param
     *reinterpret_cast<uint2 *>(orow + 16 * d + 4 * g) = o;
   }
 }
+
+static_assert(kD512Tile % kD512Rows == 0, "a workgroup's rows see the same tiles");
+static_assert(kD512Blocks == 4, "two waves' blocks are one period of V's swizzle");
 
 bool prefill_args_ok(const void *out, const void *qp, const void *kp, const void *vp,
                      const void *q, const void *k, const void *position, int batch_size,
@@ -492,8 +800,11 @@ extern "C" hipError_t gemma4_flash_attention_global_fwd_bf16_norm_rope(
   ap.v = reinterpret_cast<const uint16_t *>(d_v_prepared);
   ap.seq_len = seqlen_q;
   ap.q_scale = softmax_scale * kLog2e;
-  hipLaunchKernelGGL(prefill_d512_kernel,
-                     dim3((seqlen_q + kD512Rows - 1) / kD512Rows, batch_size),
-                     dim3(kD512Threads), 0, stream, ap);
+  const dim3 grid((seqlen_q + kD512Rows - 1) / kD512Rows, batch_size);
+  if (seqlen_q <= kD512ShortRows) {
+    hipLaunchKernelGGL(prefill_d512_short_kernel, grid, dim3(kD512ShortThreads), 0, stream, ap);
+  } else {
+    hipLaunchKernelGGL(prefill_d512_kernel, grid, dim3(kD512Threads), 0, stream, ap);
+  }
   return hipGetLastError();
 }

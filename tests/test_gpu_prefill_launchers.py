@@ -178,3 +178,34 @@ def test_launcher_argument_checks(dev):
     nulls = [None] + [z] * 10
     assert gk.flash_attention_global_fwd_bf16_norm_rope(*nulls, 1, 4, 4, 0.1) != 0
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("batch,seq,weight", [
+    (1, 256, 1.0), (1, 257, 1.0), (2, 260, 8.0), (1, 287, 8.0), (1, 289, 1.0), (3, 320, 8.0), (1, 1030, 8.0)])
+def test_global_long_and_short_forms(dev, batch, seq, weight):
+    """Both 1 x 512 kernels around the length that separates them, at the
+    edges of row groups and key tiles, against fp64 attention over the GPU's
+    own prepared rows; large norm weights make scores whose running maximum
+    moves in many tiles."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(seq)
+
+    def rnd(*shape):
+        return torch.randn(shape, generator=gen, device=dev).bfloat16()
+    q, k = rnd(batch, seq, QH, 512), rnd(batch, seq, 1, 512)
+    w = torch.full((512,), weight, device=dev).bfloat16()
+    cos, sin = torch.ones((seq, 64), device=dev), torch.zeros((seq, 64), device=dev)
+    pos = torch.arange(seq, dtype=torch.int32, device=dev).repeat(batch)
+    qp, kp, vp = torch.empty_like(q), torch.empty_like(k), torch.empty_like(k)
+    out = torch.full_like(q, float("nan"))
+    scale = 1 / math.sqrt(512)
+    gk.check(gk.flash_attention_global_fwd_bf16_norm_rope(
+        out, qp, kp, vp, q, k, w, torch.ones_like(w), cos, sin, pos, batch, seq, seq, scale))
+    hidden = torch.ones((seq, seq), dtype=torch.bool, device=dev).triu(1)
+    for b in range(batch):
+        s = qp[b].double().permute(1, 0, 2) @ kp[b, :, 0].double().T * scale
+        p = torch.softmax(s.masked_fill(hidden, -math.inf), -1)
+        exp = (p @ vp[b, :, 0].double()).permute(1, 0, 2)
+        # bf16 probabilities and one output rounding: 2^-9 of the weighted |V|, 2^-9 of the value.
+        bound = 2.0 ** -8 * (p @ vp[b, :, 0].double().abs()).permute(1, 0, 2) + 2.0 ** -8 * exp.abs()
+        assert bool(((out[b].double() - exp).abs() <= bound).all()), (b, seq)
