@@ -639,7 +639,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   next_valid = prepare_copy(tile0, phys0, ksrc, vsrc);
   issue_copies(Stage<1>{});  // into stage 0
   copy_dwords(page_entry(tile0 + 2 * kTileKeys), page_dst[0]);
-  next_valid = prepare_copy(tile0 + kTileKeys, phys1, ksrc, vsrc);
+  if (n_tiles > 1) next_valid = prepare_copy(tile0 + kTileKeys, phys1, ksrc, vsrc);
   auto step = [&](auto st, int it) __attribute__((always_inline)) {
     constexpr int S = decltype(st)::value;
     const int kt = tile0 + it * kTileKeys;
