@@ -24,52 +24,75 @@ constexpr int kNormThreads = 512;
 constexpr int kHiddenPacks = kHidden / kPackElems;  // 480
 static_assert(kHiddenPacks <= kNormThreads, "one pack per norm thread");
 
-// One row of width 4096: v_dot2 GEMV. A wave owns kCols hidden columns and
-// holds all of their weights in registers (32 16-byte packs per lane, each
-// load instruction reading 1 KiB of one column's contiguous weights): lane l
-// dots packs l, l + 64, ... (exact bf16 products, one rounding per pair) and a
-// wave sum finishes each column. 7.5 us against 7.9 on the MFMA kernel, which
-// is as fast or faster from two rows on and at width 8192 (12.0 against 12.5).
+// Few rows (kFewRows): v_dot2 GEMV. A wave owns kCols hidden columns and holds
+// all of their weights in registers (32 16-byte packs per lane, each load
+// instruction reading 1 KiB of one column's contiguous weights), then runs
+// each row against them: lane l dots packs l, l + 64, ... (exact bf16
+// products, one rounding per pair) and a wave sum finishes each column.
 constexpr int kRowWaves = 4;
-constexpr int kRowWidth = 4096;
-constexpr int kPacks = kRowWidth / (kPackElems * kWave);  // per lane per column
-constexpr int kCols = 32 / kPacks;                        // 32 packs in flight per lane
-static_assert(kCols == 4 && kHidden % (kCols * kRowWaves) == 0, "whole column groups");
 
-__global__ __launch_bounds__(kRowWaves *kWave) void o_projection_row_kernel(
+template <int kWidth>
+struct RowShape {
+  static constexpr int kPacks = kWidth / (kPackElems * kWave);  // per lane per column
+  static constexpr int kCols = 32 / kPacks;                     // 32 packs in flight per lane
+  static constexpr int kGroups = kHidden / (kCols * kRowWaves);
+  // The most rows that this kernel takes. Projection + tail with the weights
+  // streamed from HBM, here and on the MFMA kernel: width 4096, 1 / 2 / 3 / 4
+  // rows 9.4 / 10.2 / 10.9 / 11.6 us against - / 11.0 / 11.2 / 11.3; width
+  // 8192, 1 / 2 / 4 / 6 rows 14.1 / 15.4 / 18.0 / 19.9 against 18.8 / 18.9 /
+  // 19.0 / 19.0 (with the weights in the Infinity Cache the MFMA kernel is
+  // level at one row, but a model's layers do not fit there).
+  static constexpr int kFewRows = kWidth == 4096 ? 3 : 4;
+  static_assert(kWidth % (kPackElems * kWave) == 0 && 32 % kPacks == 0, "width");
+  static_assert(kHidden % (kCols * kRowWaves) == 0, "whole column groups");
+};
+
+template <int kWidth>
+__global__ __launch_bounds__(kRowWaves *kWave) void o_projection_rows_kernel(
     const uint16_t *__restrict__ attn, const uint16_t *__restrict__ w,
-    uint16_t *__restrict__ residual) {
+    uint16_t *__restrict__ residual, int32_t rows) {
+  using S = RowShape<kWidth>;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = wave_uniform(threadIdx.x / kWave);
-  const int col0 = (blockIdx.x * kRowWaves + wave) * kCols;
-  uint4 wp[kCols][kPacks];
+  const int col0 = (blockIdx.x * kRowWaves + wave) * S::kCols;
+  uint4 wp[S::kCols][S::kPacks];
 #pragma unroll
-  for (int c = 0; c < kCols; ++c)
+  for (int c = 0; c < S::kCols; ++c)
 #pragma unroll
-    for (int i = 0; i < kPacks; ++i)
-      wp[c][i] = load128_stream(w + (int64_t)(col0 + c) * kRowWidth + (i * kWave + lane) * kPackElems);
-  uint4 ap[kPacks];
+    for (int i = 0; i < S::kPacks; ++i)
+      wp[c][i] = load128_stream(w + (int64_t)(col0 + c) * kWidth + (i * kWave + lane) * kPackElems);
+  for (int32_t r = 0; r < rows; ++r) {
+    const uint16_t *a = attn + (int64_t)r * kWidth;
+    uint4 ap[S::kPacks];
 #pragma unroll
-  for (int i = 0; i < kPacks; ++i) ap[i] = load128(attn + (i * kWave + lane) * kPackElems);
-  float sum[kCols];
+    for (int i = 0; i < S::kPacks; ++i) ap[i] = load128(a + (i * kWave + lane) * kPackElems);
+    float sum[S::kCols];
 #pragma unroll
-  for (int c = 0; c < kCols; ++c) {
-    float s = 0.0f;
+    for (int c = 0; c < S::kCols; ++c) {
+      float s = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kPacks; ++i) {
-      s = dot2_bf16(ap[i].x, wp[c][i].x, s);
-      s = dot2_bf16(ap[i].y, wp[c][i].y, s);
-      s = dot2_bf16(ap[i].z, wp[c][i].z, s);
-      s = dot2_bf16(ap[i].w, wp[c][i].w, s);
+      for (int i = 0; i < S::kPacks; ++i) {
+        s = dot2_bf16(ap[i].x, wp[c][i].x, s);
+        s = dot2_bf16(ap[i].y, wp[c][i].y, s);
+        s = dot2_bf16(ap[i].z, wp[c][i].z, s);
+        s = dot2_bf16(ap[i].w, wp[c][i].w, s);
+      }
+      sum[c] = wave_sum(s);
     }
-    sum[c] = wave_sum(s);
+    if (lane == 0) {
+      uint16_t *out = residual + (int64_t)r * kHidden + col0;
+      if constexpr (S::kCols == 4) {
+        *reinterpret_cast<uint2 *>(out) =
+            make_uint2(pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3]));
+      } else {
+        *reinterpret_cast<uint32_t *>(out) = pack_bf16x2(sum[0], sum[1]);
+      }
+    }
   }
-  if (lane == 0)
-    *reinterpret_cast<uint2 *>(residual + col0) =
-        make_uint2(pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3]));
 }
 
-// Otherwise: D[row][col] = sum_k attn[row][k] * W[col][k] on v_mfma_f32_16x16x32_bf16. Workgroup: kColBlocks x 16 hidden columns and
+// Otherwise: D[row][col] = sum_k attn[row][k] * W[col][k] on
+// v_mfma_f32_16x16x32_bf16. Workgroup: kColBlocks x 16 hidden columns and
 // kRowBlocks x 16 rows; its four waves split k and work on their own until
 // the partial sums meet in LDS. In a step lane l supplies A = attn[row l % 16]
 // [k0 + 8 (l / 16) ..] and B = W[col l % 16][the same k], one 16-byte pack
@@ -276,9 +299,10 @@ hipError_t launch_blocks(const uint16_t *attn, const uint16_t *w, uint16_t *resi
 template <int kWidth>
 hipError_t launch_projection(const uint16_t *attn, const uint16_t *w, uint16_t *residual,
                              int32_t rows, hipStream_t stream) {
-  if (rows == 1 && kWidth == kRowWidth) {
-    hipLaunchKernelGGL(o_projection_row_kernel, dim3(kHidden / (kCols * kRowWaves)),
-                       dim3(kRowWaves * kWave), 0, stream, attn, w, residual);
+  using S = RowShape<kWidth>;
+  if (rows <= S::kFewRows) {
+    hipLaunchKernelGGL(o_projection_rows_kernel<kWidth>, dim3(S::kGroups), dim3(kRowWaves * kWave),
+                       0, stream, attn, w, residual, rows);
     return hipGetLastError();
   }
   if (rows <= 16) return launch_blocks<kWidth, 1, 1>(attn, w, residual, rows, stream);

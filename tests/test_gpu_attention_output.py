@@ -109,7 +109,7 @@ def test_o_projection_argument_checks(dev):
 
 
 @pytest.mark.parametrize("rows,width", [
-    (2, 4096), (2, 8192), (16, 4096), (32, 8192), (33, 4096), (64, 8192), (65, 4096), (96, 4096),
+    (3, 4096), (4, 4096), (4, 8192), (5, 8192), (16, 4096), (32, 8192), (33, 4096), (64, 8192), (65, 4096), (96, 4096),
     (97, 4096), (128, 4096), (129, 4096), (192, 4096), (193, 4096), (256, 4096), (257, 4096), (131, 8192)])
 def test_o_projection_block_edges(dev, rows, width):
     """Every split into row and column blocks at its edges, against the fp64
