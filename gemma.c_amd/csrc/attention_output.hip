@@ -103,9 +103,13 @@ __global__ __launch_bounds__(kRowWaves *kWave) void o_projection_rows_kernel(
 // operands come through LDS: 64 k (one 128-byte line) of 8 rows per copy
 // instruction, into a ring of the wave's own; chunk c of row r at
 // c ^ (r / 2 % 8), which keeps the operand reads free of bank conflicts.
-// Projection + tail at width 8192, before and now: 8 rows 20.9 -> 14.8 us, 24
-// 30.5 -> 15.1 (kernel 26.2 -> 13.0: 4.9 TB/s of weights), 64 50 -> 21.5, 256
-// 155 -> 37; width 4096, 64 rows 27.6 -> 11.7, 256 81 -> 18.6.
+// Projection + tail, before and now, weights from HBM: width 8192, 8 rows
+// 21.2 -> 19.1 us, 24 28.1 -> 20.8, 64 44.9 -> 25.6, 128 78 -> 31.6; width
+// 4096, 8 rows 12.9 -> 11.6, 64 25.1 -> 15.5, 128 39.8 -> 18.9. With four
+// copies of the weights in turn, which the 256 MiB Infinity Cache still helps:
+// width 8192, 24 rows 30.5 -> 15.1 (kernel 26.2 -> 13.0), 256 155 -> 37.
+// Nontemporal weight copies gain 1-2 us from HBM up to 24 rows (8192, 8 rows
+// 17.1) but give up that help (24 rows 19.0 against 15.1), and lose from 64 rows on.
 constexpr int kSplit = 4;  // waves per workgroup, one k slice each
 constexpr int kChunkK = 64;
 constexpr int kBlockUint4 = 16 * kChunkK / kPackElems;  // 16 rows of a chunk: 2 KiB

@@ -900,8 +900,8 @@ hipError_t decode_entry(uint16_t *out, float *pm, float *pl, float *pacc,
   const bool d512 = c.head_dim == 512;
   // A batch whose combine follows is cut by its lengths (balanced_cut): two
   // workgroups per CU, all resident at once. Not one that takes a single
-  // round of one-step workgroups as planned (2 x 500-1000 keys: 12.4 against 17 us). One sequence is planned by its
-  // length already, except in a step (gate), which plans by the cache's
+  // round of one-step workgroups as planned (2 x 500-1000 keys: 12.4 against
+  // 17 us). One sequence is planned by its length already, except in a step (gate), which plans by the cache's
   // capacity: a cut there once that gives splits of more than one step.
   const bool one_round = split_size <= kD512OneStep && (int64_t)num_splits * batch_count <= kD512Cus;
   if (d512 && combine && p.counters == nullptr && num_splits > 1 && batch_count <= kBalancedBatch &&

@@ -422,8 +422,8 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
 
   // Row addresses of a tile: lane j < 16 resolves key 16w + j and publishes
   // {K row, V row} in the wave's row table (the readable-key bits are
-  // returned: the tile's stage is still in use); lane l then fetches key 16w + 2a + l/32 of copy a and adds its
-  // swizzled source chunk.
+  // returned: the tile's stage is still in use); lane l then fetches key
+  // 16w + 2a + l/32 of copy a and adds its swizzled source chunk.
   auto prepare_copy = [&](int kt, int32_t phys, uint64_t (&ksrc)[kCopyKeys / 2],
                           uint64_t (&vsrc)[kCopyKeys / 2]) __attribute__((always_inline)) -> uint32_t {
     uint4 rows;

@@ -207,8 +207,8 @@ hipError_t gemma4_flash_attention_global_fwd_bf16_norm_rope(
 
 // Split plan for the MI355X: the split size (a multiple of the kernel's key
 // wave chunk) that gives about `target_workgroups` split workgroups (0 = default:
-// one per CU for one sequence, 32 per CU for a batch) for `batch_count` sequences of up to `max_live_keys` live keys,
-// and the split count that covers `max_live_keys`. With the default target,
+// one per CU for one sequence, 32 per CU for a batch) for `batch_count`
+// sequences of up to `max_live_keys` live keys, and the split count that covers `max_live_keys`. With the default target,
 // one sequence whose splits would hold two key tiles or fewer (a 1024-key
 // sliding window) gets one-tile splits instead, up to two workgroups per CU;
 // a batch's splits at 1 x 512 hold 96 keys at least (its combining launches
