@@ -500,10 +500,20 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
     }
     // A probability is the sum of two bf16, 16 bits of it: one bf16 alone left
     // the outputs further from the 64-bit result than shorter splits did
-    // (whose largest weights are 1), and the matrix units have the room.
-    const uint32_t hi01 = cvt_pk_bf16(pr[0], pr[1]), hi23 = cvt_pk_bf16(pr[2], pr[3]);
-    s_p[wave][lane] = make_uint4(hi01, hi23, cvt_pk_bf16(pr[0] - bf16_lo(hi01), pr[1] - bf16_hi(hi01)),
-                                 cvt_pk_bf16(pr[2] - bf16_lo(hi23), pr[3] - bf16_hi(hi23)));
+    // (whose largest weights are 1), and the matrix units have the room. Both
+    // parts are positive (the first is cut, not rounded, and the rest is
+    // 2^-126 at least): with a negative or zero second part an infinite V
+    // would turn into NaN.
+    auto upper = [](float a, float b) __attribute__((always_inline)) {
+      return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+    };
+    const uint32_t hi01 = upper(pr[0], pr[1]), hi23 = upper(pr[2], pr[3]);
+    const float hi[4] = {bf16_lo(hi01), bf16_hi(hi01), bf16_lo(hi23), bf16_hi(hi23)};
+    float lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lo[i] = fmaxf(pr[i] - hi[i], fminf(pr[i], 0x1p-126f));
+    s_p[wave][lane] =
+        make_uint4(hi01, hi23, cvt_pk_bf16(lo[0], lo[1]), cvt_pk_bf16(lo[2], lo[3]));
 
     if (live_next) {
       wait_vector<kTileKeys>();  // V of this step (the next K copies are younger)

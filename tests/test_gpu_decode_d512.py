@@ -151,3 +151,26 @@ def test_step_plans_by_capacity(dev):
     assert gk.decode_step_status(ws) == 0
     assert np.array_equal(from_dev_bf16(ck).reshape(exp_k.shape), exp_k)
     assert_close(from_dev_bf16(out), exp, "capacity plan")
+
+
+@pytest.mark.parametrize("split,seq", [
+    (64, [300]),               # one-step splits, four waves
+    (160, [450]),              # several steps, two waves
+    (512, [200]),              # a single split
+    (200, [150, 700, 31]),     # cut by the lengths
+])
+def test_infinite_values(dev, split, seq):
+    """An infinite V element of one live key makes its dim infinite, with its
+    sign, in every head; all others stay finite and right."""
+    rng = np.random.default_rng(split + 7)
+    cfg, pt, ck, cv, q, splits = _case(rng, split, seq, 0, 16)
+    max_pages = cfg[3]
+    for b, n in enumerate(seq):
+        for key, dim, bits in ((n // 2, 5, 0x7F80), (n - 1, 200, 0xFF80), (0, 511, 0x7F80)):
+            cv[pt[b * max_pages + key // 16] * 16 + key % 16, 0, dim] = bits
+    exp = oracle.decode_attention(q, ck, cv, pt, seq, cfg, 0, 0.0442)
+    got = _run_decode(dev, cfg, q, to_dev(ck, dev), to_dev(cv, dev), pt, seq, 0, 0.0442, split, splits)
+    infinite = (exp & 0x7FFF) == 0x7F80
+    assert infinite.sum() == 3 * 16 * len(seq)
+    assert np.array_equal(got[infinite], exp[infinite])
+    assert_close(np.where(infinite, 0, got), np.where(infinite, 0, exp), "finite dims")
