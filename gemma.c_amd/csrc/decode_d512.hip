@@ -193,7 +193,10 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   const int32_t token_pos = p.token_position != nullptr ? wave_uniform(tok_word) : -1;
   int32_t first = c.window_size > 0 ? seq_len - c.window_size : 0;
   first = first < 0 ? 0 : first;
-  const int32_t key_count = seq_len > first ? seq_len - first : 0;
+  // The plan's splits bound the keys, however the launch cuts them.
+  const int32_t capacity =
+      (int32_t)min((int64_t)p.split_size * p.num_splits, (int64_t)0x7fffffff);
+  const int32_t key_count = min(seq_len > first ? seq_len - first : 0, capacity);
   const int32_t live_splits = (key_count + split_size - 1) / split_size;
   const bool direct = p.num_splits == 1;
 
@@ -256,7 +259,7 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
 
   // ---- steps; the last ones of the split may leave waves without a key
   const int32_t begin = first + split * split_size;
-  const int32_t end = min(seq_len, begin + split_size);
+  const int32_t end = min(first + key_count, begin + split_size);
   const int32_t n_tiles = (end - begin + kTileKeys - 1) / kTileKeys;
   const int32_t n_steps = (n_tiles + kWaves - 1) / kWaves;
   // Key of lane (tile within the lookup, h) of lookup m, at most end - 1.

@@ -174,3 +174,19 @@ def test_infinite_values(dev, split, seq):
     assert infinite.sum() == 3 * 16 * len(seq)
     assert np.array_equal(got[infinite], exp[infinite])
     assert_close(np.where(infinite, 0, got), np.where(infinite, 0, exp), "finite dims")
+
+
+def test_keys_past_the_plan_are_not_attended_to(dev):
+    """A plan of fewer keys than a sequence holds covers the first split_size *
+    num_splits of them, in a batch cut by its lengths as in a single sequence."""
+    rng = np.random.default_rng(81)
+    seq, split, splits = [700, 150, 310], 70, 3
+    cfg, pt, ck, cv, q, _ = _case(rng, split, seq, 0, 16)
+    covered = [min(n, split * splits) for n in seq]
+    exp = oracle.decode_attention(q, ck, cv, pt, covered, cfg, 0, 0.0442)
+    got = _run_decode(dev, cfg, q, to_dev(ck, dev), to_dev(cv, dev), pt, seq, 0, 0.0442, split, splits)
+    assert_close(got, exp, "batch")
+    one = cache_config(1, 1, 16, cfg[3], 1, 512, 0)
+    got = _run_decode(dev, one, q[:1], to_dev(ck, dev), to_dev(cv, dev), pt[:cfg[3]], seq[:1], 0, 0.0442, split,
+                      splits)
+    assert_close(got, exp[:1], "single")
