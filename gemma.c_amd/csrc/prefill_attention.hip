@@ -802,7 +802,8 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillP
     }
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const float mi = i0 + i < live_parts ? pm[i] : -INFINITY;
+      if (i0 + i >= live_parts) break;  // a repeated part: 0 * infinity is not 0
+      const float mi = pm[i];
       const float m_new = fmaxf(m, mi);
       const float fa = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
       const float fb = mi == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mi - m_new);

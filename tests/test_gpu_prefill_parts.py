@@ -86,3 +86,35 @@ def test_workspace_bytes_never_shrink_with_the_call():
     for n in (1, 64, 65, 512, 1024, 1025, 2048):
         sizes = [gk.flash_attention_prefill_chunk_workspace_bytes(b, n, c) for b in (1, 2, 4)]
         assert sizes == sorted(sizes) and sizes[-1] <= largest
+
+
+@pytest.mark.parametrize("prior,lq", [(600, 40), (129, 64), (1537, 100)])
+def test_infinite_values(dev, prior, lq):
+    """An infinite V element of the last cached key, which every row sees, in
+    the last part of a row block: infinite in that dim, finite and right
+    elsewhere."""
+    import torch
+    rng = np.random.default_rng(prior)
+    page = 16
+    max_pages = (prior + lq) // page + 1
+    cfg = cache_config(1, 1, page, max_pages, H, D, 0)
+    q, k, v = (randn_bf16(rng, (1, lq, h, D)) for h in (16, H, H))
+    ck, cv = (randn_bf16(rng, (max_pages * page, H, D)) for _ in range(2))
+    pt = fill_page_table(cfg, [prior])
+    pos = np.arange(prior)
+    r = pt[pos // page].astype(np.int64) * page + pos % page
+    cv[r[-1], :, 7], cv[r[-1], :, 250] = 0x7F80, 0xFF80
+    c = gk.make_config(*cfg)
+    need = gk.flash_attention_prefill_chunk_workspace_bytes(1, lq, c)
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    out = empty_bf16((1, lq, 16, D), dev)
+    gk.check(gk.flash_attention_prefill_chunk_paged_bf16_ws(
+        out, *(to_dev(x, dev) for x in (q, k, v, ck, cv, pt, np.int32([prior]))), c, 0, 1, lq, 1 / 16, ws, need))
+    torch.cuda.synchronize()
+    got = from_dev_bf16(out)
+    finite = np.where((cv & 0x7FFF) == 0x7F80, 0, cv)
+    full = [np.concatenate([c0[r], new[0]])[None] for c0, new in ((ck, k), (finite, v))]
+    exp = oracle.prefill_attention(q, *full, lq, prior + lq, 16, H, D, 0, 1 / 16)
+    assert (got[..., 7] == 0x7F80).all() and (got[..., 250] == 0xFF80).all()
+    rest = [d for d in range(D) if d not in (7, 250)]
+    assert_close(got[..., rest], exp[..., rest], "finite dims")
