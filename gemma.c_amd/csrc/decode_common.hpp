@@ -172,14 +172,10 @@ __device__ __forceinline__ int32_t append_row(const Gemma4KvCacheConfig &c,
   return key_row(c, page_table, layer, b, position);
 }
 
-// Device-coherent (sc1) accesses for data exchanged between workgroups of
-// one launch: they bypass the per-XCD L2 write-back state, so no whole-cache
-// maintenance is needed (agent-scope relaxed atomics compile to the same).
-constexpr int kCoherentAux = 16;  // cache-policy bit sc1
+// Device-coherent accesses (kCoherentAux).
 __device__ __forceinline__ void coherent_store(float *p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 // 8 floats at byte offset `off` (per lane) from the wave-uniform `base`: a
 // buffer descriptor must be uniform, or the compiler loops over the lanes.
 __device__ __forceinline__ void coherent_store8(float *base, int32_t off, const float (&v)[8]) {
@@ -191,14 +187,6 @@ __device__ __forceinline__ void coherent_store8(float *base, int32_t off, const 
   __builtin_amdgcn_raw_buffer_store_b128(lo, rsrc, off, 0, kCoherentAux);
   __builtin_amdgcn_raw_buffer_store_b128(hi, rsrc, off + 16, 0, kCoherentAux);
 }
-// Wait until this thread's outstanding memory operations have completed
-// (the signal fences keep the compiler from moving memory accesses across).
-__device__ __forceinline__ void wait_stores_complete() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0);
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
 // Buffer view of `count` floats for coherent loads; out-of-range loads read 0.
 __device__ __forceinline__ auto coherent_view(const float *p, int32_t count) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, count * 4, 0x00020000);

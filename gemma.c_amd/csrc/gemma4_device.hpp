@@ -198,4 +198,17 @@ __device__ __forceinline__ int32_t wave_uniform(int32_t v) {
   return __builtin_amdgcn_readfirstlane(v);
 }
 
+// Device-coherent (sc1) accesses for data exchanged between workgroups of
+// one launch: they bypass the per-XCD L2 write-back state, so no whole-cache
+// maintenance is needed (agent-scope relaxed atomics compile to the same).
+constexpr int kCoherentAux = 16;  // cache-policy bit sc1
+using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
+// Wait until this thread's outstanding memory operations have completed
+// (the signal fences keep the compiler from moving memory accesses across).
+__device__ __forceinline__ void wait_stores_complete() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
 }  // namespace gemma4

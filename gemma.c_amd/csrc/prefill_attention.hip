@@ -98,12 +98,13 @@ struct PrefillParams {
   int32_t n_pairs;
   char *ws;
   // Chunks of few row blocks (n_parts > 1): every row block's key tiles are
-  // shared out over up to n_parts workgroups, whose partials a second launch
-  // merges.
+  // shared out over up to n_parts workgroups, which merge their partials.
   int32_t n_parts;
 };
 
 enum class Mode { kPlain, kPaired, kParts };
+
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kPartialFloats = 130;  // per thread: 128 accumulators, max, sum
 // Workspace slot s at s * kSlotBytes: the arrival counter (256-byte
@@ -119,10 +120,11 @@ __device__ __forceinline__ float *part_partial(char *ws, int64_t i) {
   return reinterpret_cast<float *>(ws + (i >> 1) * kSlotBytes + kSlotCounterBytes +
                                    (i & 1) * kPartialBytes);
 }
-// A row block's share of `tiles` key tiles in parts: tiles per part, two at
-// least (a workgroup's start costs as much as five tiles).
+// A row block's share of `tiles` key tiles in parts: tiles per part. One tile
+// is worth a workgroup of its own (64 rows after 37 keys, two tiles: in one
+// part 13.6 us, in two 11.6).
 __device__ __forceinline__ int part_tiles(int tiles, int n_parts) {
-  return max((tiles + n_parts - 1) / n_parts, 2);
+  return tiles <= n_parts ? 1 : (tiles + n_parts - 1) / n_parts;
 }
 // Key tiles of causal row block blk (no window).
 __device__ __forceinline__ int causal_tiles(int prior, int chunk_len, int blk) {
@@ -217,6 +219,160 @@ __device__ __forceinline__ void static_for(F &&f) {
 template <int kSt>
 using Stage = std::integral_constant<int, kSt>;
 
+// Partial of a row block in parts: 32 columns of four accumulators, float4
+// [column][thread], then {maximum, sum} [thread]. Stored and loaded
+// device-coherently: a row block's workgroups may run on different XCDs.
+constexpr int kPartColumns = 32;
+__device__ __forceinline__ auto part_view(char *ws, int64_t i, int offset, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(
+      reinterpret_cast<char *>(part_partial(ws, i)) + offset, 0, bytes, 0x00020000);
+}
+// Byte offset of this thread in column 0. The empty asm keeps what is derived
+// from it out of the registers of the loop over the keys.
+__device__ __forceinline__ int part_thread() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t * 16;
+}
+constexpr int kPartColumnBytes = kPrefillThreads * 16;
+constexpr int kPartStats = kPartColumns * kPartColumnBytes;  // byte offset
+
+// Columns c0 .. c0 + n - 1 (n <= kColumns) of this thread over the parts from
+// `part0` on, kBatch parts' loads at a time, into its output row. Loads past
+// the columns and past the parts are out of their view's range: they read 0
+// and move nothing, so nothing branches between the loads of a batch.
+template <int kColumns, int kBatch>
+__device__ __forceinline__ void merge_columns(char *ws, int64_t part0, int live_parts, int c0,
+                                              int n, uint16_t *orow) {
+  const int off = part_thread();
+  float m = -INFINITY, l = 0.0f;
+  float acc[kColumns][4] = {};
+  for (int i0 = 0; i0 < live_parts; i0 += kBatch) {
+    u32x2 stats[kBatch];
+    u32x4 a[kBatch][kColumns];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const bool live = i0 + i < live_parts;
+      const int64_t part = part0 + (live ? i0 + i : 0);
+      stats[i] = __builtin_amdgcn_raw_buffer_load_b64(
+          part_view(ws, part, kPartStats, live ? kPrefillThreads * 8 : 0), off / 2, 0,
+          kCoherentAux);
+      const auto columns =
+          part_view(ws, part, c0 * kPartColumnBytes, live ? n * kPartColumnBytes : 0);
+#pragma unroll
+      for (int c = 0; c < kColumns; ++c)
+        a[i][c] = __builtin_amdgcn_raw_buffer_load_b128(columns, off + c * kPartColumnBytes, 0,
+                                                        kCoherentAux);
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const float mi = i0 + i < live_parts ? __uint_as_float(stats[i][0]) : -INFINITY;
+      const float m_new = fmaxf(m, mi);
+      const float fa = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+      const float fb = mi == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mi - m_new);
+      l = l * fa + __uint_as_float(stats[i][1]) * fb;
+#pragma unroll
+      for (int c = 0; c < kColumns; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[c][e] = acc[c][e] * fa + __uint_as_float(a[i][c][e]) * fb;
+      m = m_new;
+    }
+  }
+  // Lanes l and l ^ 32 hold one row's sums over different keys (and share
+  // the maximum). Both are here: they have the same row.
+  l = xor_sum<32>(l);
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const int half = (threadIdx.x & 63) >> 5;
+#pragma unroll
+  for (int c = 0; c < kColumns; ++c) {
+    if (c >= n) break;
+    // Column: accumulators 16 d + 4 i .. + 3, dims 32 d + 8 i + 4 half ..
+    *reinterpret_cast<uint2 *>(orow + 8 * (c0 + c) + 4 * half) =
+        make_uint2(pack_bf16x2(acc[c][0] * inv, acc[c][1] * inv),
+                   pack_bf16x2(acc[c][2] * inv, acc[c][3] * inv));
+  }
+}
+
+// The end of a row block in parts: its n_parts workgroups, the ones without
+// keys included, call this (after storing their partials, if they have one)
+// and merge the partials together, each its share of the columns. The first
+// word of the block's slot counts the workgroups that have stored (low half);
+// another counts those that have left, and the last of them sets both to zero.
+// A workgroup waits for the others a bounded time only; then it marks its
+// share (high half of the first word) and leaves. The last to store waits for
+// nobody and also merges the marked shares, so the rows are written whatever
+// else runs on the GPU. The partials are folded in part order: the result does
+// not depend on who merges.
+// A second launch for the merge, as before, was paid for by every chunk, also
+// if its row blocks are one part each: the device knows that, the host does
+// not. 64 rows after 0 / 37 / 300 keys in a cache of 8192: 12.8 / 15.1 / 13.9
+// -> 11.3 / 11.6 / 13.0 us (plain form 11.05 / 13.1 / 20.9); 93 rows after 7401
+// 32.9 -> 31.6. The workgroups without keys matter: merged by the others alone
+// 64 rows after 300 took 16.5. So does little code, which runs once, cold:
+// eight columns and four parts unrolled, 18.4.
+constexpr uint64_t kMergeWaitTicks = 200;  // per tile of a part: 2 us at 100 MHz
+__device__ __forceinline__ void merge_parts(const PrefillParams &p, int b, int blk, int head,
+                                            int part, int live_parts, int tiles,
+                                            uint64_t *s_word) {
+  const int t = threadIdx.x;
+  const int64_t block =
+      ((int64_t)b * ((p.chunk_len + kPrefillRows - 1) / kPrefillRows) + blk) * p.c.num_heads + head;
+  auto *const word = reinterpret_cast<unsigned long long *>(p.ws + block * kSlotBytes);
+  auto *const left = reinterpret_cast<int32_t *>(word + 1);
+  wait_stores_complete();
+  __syncthreads();
+  if (t == 0) {
+    auto all_stored = [&](unsigned long long w) { return (uint32_t)w == (uint32_t)live_parts; };
+    const uint64_t limit = __builtin_amdgcn_s_memrealtime() + kMergeWaitTicks * (tiles + 16);
+    bool last = false;
+    unsigned long long w;
+    if (part < live_parts) {
+      w = 1 + __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = all_stored(w);
+    } else {
+      w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    while (!all_stored(w) && __builtin_amdgcn_s_memrealtime() < limit) {
+      __builtin_amdgcn_s_sleep(2);
+      w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!all_stored(w))
+      w = __hip_atomic_fetch_or(word, 1ull << (32 + part), __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+    // The shares to merge: this workgroup's if all have stored, and the marked
+    // ones if it was the last.
+    uint32_t shares = all_stored(w) ? 1u << part : 0;
+    if (last) shares |= (uint32_t)(w >> 32);
+    *s_word = shares;
+  }
+  __syncthreads();
+  const int lane = t & 63, n = lane & 31;
+  const int row = blk * kPrefillRows + 16 * (t >> 6) + n % 16;
+  if (row < p.chunk_len) {
+    const int qh = head * (kQueryHeads / p.c.num_heads) + n / 16;
+    uint16_t *orow = p.out + (((int64_t)b * p.chunk_len + row) * kQueryHeads + qh) * kDim;
+    uint32_t shares = (uint32_t)wave_uniform((int32_t)*s_word);
+    for (; shares != 0; shares &= shares - 1) {
+      const int i = __builtin_ctz(shares);
+      const int end = kPartColumns * (i + 1) / p.n_parts;
+      int c0 = kPartColumns * i / p.n_parts;
+      if (p.n_parts <= 4) {
+        for (; c0 < end; c0 += 8)
+          merge_columns<8, 2>(p.ws, block * p.n_parts, live_parts, c0, min(end - c0, 8), orow);
+      } else {
+        for (; c0 < end; c0 += 2)
+          merge_columns<2, 4>(p.ws, block * p.n_parts, live_parts, c0, min(end - c0, 2), orow);
+      }
+    }
+  }
+  if (t == 0 && __hip_atomic_fetch_add(left, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                    p.n_parts - 1) {
+    __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(left, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 template <Mode kMode>
 __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(PrefillParams p) {
   constexpr int KS = kDim / 16;        // k-steps of S^T (dims)
@@ -267,18 +423,21 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   constexpr int kAllTiles = 1 << 30;
   Unit unit0 = {0, 0, 0, -1, 0}, unit1 = {0, 0, 0, -1, 0};
   int n_units = 0;
-  int part = 0, live_parts = 1;
+  int part = 0, live_parts = 1, part_blk = 0, per_part = 0;
   if constexpr (kMode == Mode::kParts) {
-    const int rest = blockIdx.x / Hk;
-    const int blk = rest / p.n_parts;
-    part = rest % p.n_parts;
-    const int tiles = causal_tiles(prior, Lq, blk);
-    const int per = part_tiles(tiles, p.n_parts);
-    live_parts = (tiles + per - 1) / per;
-    if (part >= live_parts) return;
-    unit0 = {kPrefillRows * blk, part * per, part == live_parts - 1 ? kAllTiles : (part + 1) * per,
-             -1, 0};
-    n_units = 1;
+    // Grid z is the part: the first parts, often the only ones, start first.
+    part = blockIdx.z;
+    part_blk = blockIdx.x / Hk;
+    const int tiles = causal_tiles(prior, Lq, part_blk);
+    per_part = part_tiles(tiles, p.n_parts);
+    live_parts = per_part == 1 ? tiles : (tiles + per_part - 1) / per_part;
+    if (part < live_parts) {
+      unit0 = {kPrefillRows * part_blk, part * per_part,
+               part == live_parts - 1 ? kAllTiles : (part + 1) * per_part, -1, 0};
+      n_units = 1;
+    } else if (live_parts == 1) {
+      return;
+    }
   } else if constexpr (kMode == Mode::kPaired) {
     const int rest = blockIdx.x / Hk;
     const int pair = rest >> 1, side = rest & 1;
@@ -312,6 +471,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
     n_units = 1;
   }
   __shared__ int s_last;
+  __shared__ uint64_t s_shares;
 
   for (int u = 0; u < n_units; ++u) {
   const Unit &cur = u == 0 ? unit0 : unit1;
@@ -674,19 +834,24 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   // second arriver merge both halves and write the rows.
   bool emit = true;
   if (kMode == Mode::kParts && live_parts > 1) {
-    // Rows past the chunk are not merged and need no partial.
     emit = false;
-    if (row_ok) {
-      const int nb = (Lq + kPrefillRows - 1) / kPrefillRows;
-      float *mine = part_partial(
-          p.ws, (((int64_t)b * nb + q0 / kPrefillRows) * Hk + head) * p.n_parts + part);
+    const int nb = (Lq + kPrefillRows - 1) / kPrefillRows;
+    const int64_t block = ((int64_t)b * nb + q0 / kPrefillRows) * Hk + head;
+    if (row_ok) {  // rows past the chunk are not merged and need no partial
+      const auto mine = part_view(p.ws, block * p.n_parts + part, 0, (int)kPartialBytes);
+      const int off = part_thread();
 #pragma unroll
       for (int d = 0; d < DB; ++d) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mine[(d * 16 + i) * kPrefillThreads + t] = acc[d][i];
+        for (int i = 0; i < 16; i += 4) {
+          const u32x4 x = {__float_as_uint(acc[d][i]), __float_as_uint(acc[d][i + 1]),
+                           __float_as_uint(acc[d][i + 2]), __float_as_uint(acc[d][i + 3])};
+          __builtin_amdgcn_raw_buffer_store_b128(x, mine, off, (4 * d + i / 4) * kPartColumnBytes,
+                                                 kCoherentAux);
+        }
       }
-      mine[128 * kPrefillThreads + t] = m_run;
-      mine[129 * kPrefillThreads + t] = l_run;
+      const u32x2 stats = {__float_as_uint(m_run), __float_as_uint(l_run)};
+      __builtin_amdgcn_raw_buffer_store_b64(stats, mine, off / 2, kPartStats, kCoherentAux);
     }
   }
   if (unit_slot >= 0) {
@@ -762,69 +927,8 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   }
   if constexpr (kMode == Mode::kPaired) __syncthreads();  // the next unit reuses the LDS stages and tables
   }  // units
-}
-
-// Merges the parts of a chunk's row blocks: workgroup (kv head, row block,
-// slice of 8 of a thread's 128 accumulators), thread t as in the chunk kernel.
-constexpr int kMergeElems = 8;
-constexpr int kMergeSlices = 128 / kMergeElems;
-__global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillParams p) {
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int Hk = p.c.num_heads;
-  const int head = blockIdx.x % Hk;
-  const int blk = blockIdx.x / Hk / kMergeSlices;
-  const int e0 = blockIdx.x / Hk % kMergeSlices * kMergeElems;
-  const int b = blockIdx.y;
-  const int Lq = p.chunk_len;
-  const int prior = p.prior != nullptr ? wave_uniform(p.prior[b]) : 0;
-  const int tiles = causal_tiles(prior, Lq, blk);
-  const int per = part_tiles(tiles, p.n_parts);
-  const int live_parts = (tiles + per - 1) / per;
-  if (live_parts == 1) return;  // the chunk kernel wrote the rows
-  const int nb = (Lq + kPrefillRows - 1) / kPrefillRows;
-  const int n = lane & 31, half = lane >> 5;
-  const int row = blk * kPrefillRows + 16 * wave + n % 16;
-  if (row >= Lq) return;
-  const int64_t part0 = (((int64_t)b * nb + blk) * Hk + head) * p.n_parts;
-  float m = -INFINITY, l = 0.0f;
-  float acc[kMergeElems] = {};
-  constexpr int kBatch = 4;  // parts whose loads go out together
-  for (int i0 = 0; i0 < live_parts; i0 += kBatch) {
-    float pm[kBatch], pl[kBatch], pa[kBatch][kMergeElems];
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      const float *part = part_partial(p.ws, part0 + min(i0 + i, live_parts - 1)) + t;
-      pm[i] = part[128 * kPrefillThreads];
-      pl[i] = part[129 * kPrefillThreads];
-#pragma unroll
-      for (int e = 0; e < kMergeElems; ++e) pa[i][e] = part[(e0 + e) * kPrefillThreads];
-    }
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      if (i0 + i >= live_parts) break;  // a repeated part: 0 * infinity is not 0
-      const float mi = pm[i];
-      const float m_new = fmaxf(m, mi);
-      const float fa = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
-      const float fb = mi == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mi - m_new);
-      l = l * fa + pl[i] * fb;
-#pragma unroll
-      for (int e = 0; e < kMergeElems; ++e) acc[e] = acc[e] * fa + pa[i][e] * fb;
-      m = m_new;
-    }
-  }
-  // Lanes l and l ^ 32 hold one row's sums over different keys (and share
-  // the maximum). Both are here: they have the same row.
-  l = xor_sum<32>(l);
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  const int qh = head * (kQueryHeads / Hk) + n / 16;
-  uint16_t *orow = p.out + (((int64_t)b * Lq + row) * kQueryHeads + qh) * kDim;
-#pragma unroll
-  for (int i = 0; i < kMergeElems; i += 4) {
-    const int d = (e0 + i) / 16, ii = (e0 + i) % 16;
-    *reinterpret_cast<uint2 *>(orow + 32 * d + (ii / 4) * 8 + 4 * half) =
-        make_uint2(pack_bf16x2(acc[i] * inv, acc[i + 1] * inv),
-                   pack_bf16x2(acc[i + 2] * inv, acc[i + 3] * inv));
+  if constexpr (kMode == Mode::kParts) {
+    if (live_parts > 1) merge_parts(p, b, part_blk, head, part, live_parts, per_part, &s_shares);
   }
 }
 
@@ -849,9 +953,9 @@ size_t prefill_workspace_bytes(int32_t batch_size, int32_t chunk_len, int32_t he
 
 // Parts per row block for a global chunk that leaves half of the 256 CUs or
 // more without a row block: as many as give every CU a workgroup, if the
-// cache (or the chunk) has room for enough keys to be worth the second
-// launch; the lengths are on the device. 93 rows after 7401 tokens: 254 -> 33 us (in
-// 15 parts of 8 tiles: the chunk launch 27, the merge 6.5).
+// cache (or the chunk) has room for enough keys; how many a row block uses is
+// settled on the device, by the length. 93 rows after 7401 tokens: 254 -> 31.6
+// us in 15 parts of 8 tiles.
 constexpr int kPartsCus = 256;
 constexpr int kPartsMinTiles = 6;
 bool parts_worthwhile(int32_t chunk_len, const Gemma4KvCacheConfig &c) {
@@ -868,7 +972,8 @@ int prefill_parts(int32_t batch_size, int32_t chunk_len, const Gemma4KvCacheConf
                   size_t workspace_bytes) {
   if (!parts_worthwhile(chunk_len, c)) return 1;
   const int64_t held = std::min<int64_t>(kPartsCus, 2 * (int64_t)(workspace_bytes / kSlotBytes));
-  return (int)std::max<int64_t>(1, held / row_blocks(batch_size, chunk_len, c.num_heads));
+  return (int)std::clamp<int64_t>(held / row_blocks(batch_size, chunk_len, c.num_heads), 1,
+                                  kPartColumns);
 }
 
 hipError_t prefill_chunk_launch(gemma4_bf16 *d_out, const gemma4_bf16 *d_q, const gemma4_bf16 *d_k,
@@ -928,11 +1033,7 @@ hipError_t prefill_chunk_launch(gemma4_bf16 *d_out, const gemma4_bf16 *d_q, cons
       usable ? prefill_parts(batch_size, chunk_len, config, workspace_bytes) : 1;
   if (parts > 1) {
     p.n_parts = parts;
-    hipLaunchKernelGGL(prefill_chunk_kernel<Mode::kParts>, dim3(blocks * parts, batch_size),
-                       dim3(kPrefillThreads), 0, stream, p);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(prefill_merge_kernel, dim3(blocks * kMergeSlices, batch_size),
+    hipLaunchKernelGGL(prefill_chunk_kernel<Mode::kParts>, dim3(blocks, batch_size, parts),
                        dim3(kPrefillThreads), 0, stream, p);
   } else if (p.n_pairs > 0) {
     hipLaunchKernelGGL(prefill_chunk_kernel<Mode::kPaired>,

@@ -154,20 +154,23 @@ hipError_t gemma4_flash_attention_prefill_chunk_paged_bf16(
     int32_t layer, int32_t batch_size, int32_t chunk_len, float softmax_scale,
     hipStream_t stream);
 
-// The same attention with the causal work of a global chunk (window 0, two
-// or more 64-row blocks) balanced over workgroups: row blocks j and nb-1-j
-// are served by two workgroups with equal key tiles, and the one block a pair
-// splits is merged through d_workspace. Results equal the entry point above
-// up to float summation order. d_workspace: at least
-// gemma4_flash_attention_prefill_chunk_workspace_bytes(batch_size,
-// chunk_len, config) bytes, 256-byte aligned, zero-filled once before its
-// first use (every call leaves its arrival counters at zero again; a
-// single row block may also come without one); one
-// sized for the largest chunk and batch also serves every smaller call;
-// calls that share a workspace must not overlap. Sliding chunks (window > 0) run
-// the plain kernel and ignore the workspace. No counterpart in the
-// reference, whose prefill launcher (src/gemma4_flash_attention_prefill.cu:
-// 1131-1183) assigns one causal row block per block.
+// The same attention with the causal work of a global chunk (window 0) shared
+// out over workgroups. A chunk of two or more 64-row blocks: row blocks j and
+// nb-1-j are served by two workgroups with equal key tiles, and the one block
+// a pair splits is merged through d_workspace. One of so few row blocks that
+// they leave half of the GPU idle: the key tiles of a row block are shared out
+// over several workgroups, which merge them through d_workspace and, where
+// they must, wait for each other for a bounded time. Results equal the entry
+// point above up to float summation order. One launch. d_workspace: at least
+// gemma4_flash_attention_prefill_chunk_workspace_bytes(batch_size, chunk_len,
+// config) bytes, 256-byte aligned, zero-filled once before its first use
+// (every call leaves its arrival counters at zero again; a single row block
+// may also come without one); one sized for the largest chunk and batch also
+// serves every smaller call; calls that share a workspace must not overlap.
+// Sliding chunks (window > 0) run the plain kernel and ignore the workspace.
+// No counterpart in the reference, whose prefill launcher
+// (src/gemma4_flash_attention_prefill.cu:1131-1183) assigns one causal row
+// block per block.
 size_t gemma4_flash_attention_prefill_chunk_workspace_bytes(
     int32_t batch_size, int32_t chunk_len, Gemma4KvCacheConfig config);
 hipError_t gemma4_flash_attention_prefill_chunk_paged_bf16_ws(

@@ -1,7 +1,8 @@
 """Global prefill chunks of few row blocks run their key tiles in parts on
-several workgroups, merged by a second launch through the workspace: the
-edges of row blocks, tiles and parts, ragged batches, smaller workspaces, and
-a balanced chunk on the same workspace afterwards."""
+several workgroups, which merge them through the workspace: the edges of row
+blocks, tiles and parts, ragged batches, unmapped pages, smaller workspaces, a
+balanced chunk on the same workspace afterwards, other work on the GPU."""
+import ctypes
 import math
 
 import numpy as np
@@ -51,10 +52,12 @@ def _run(dev, priors, lq, page, ws=None, ws_bytes=None, capacity=0):
 
 
 @pytest.mark.parametrize("priors,lq,page", [
-    ([500], 1, 16),            # one row, one row block: 32 parts of two tiles at most
-    ([0], 64, 16),             # a single part: the chunk kernel writes the rows
-    ([128 - 64], 64, 16),      # two tiles, one part
-    ([129 - 64], 64, 64),      # three tiles: parts of two and one
+    ([500], 1, 16),            # one row, one row block: eight parts of 32
+    ([0], 64, 16),             # a single part: its workgroup writes the rows
+    ([128 - 64], 64, 16),      # two tiles
+    ([129 - 64], 64, 64),      # three tiles
+    ([2047], 1, 16),           # 32 tiles for 32 parts
+    ([2048], 1, 16),           # 33: 17 parts, the last of one tile
     ([900], 63, 1),
     ([700], 65, 16),           # the second row block holds one row
     ([3, 1200, 400], 17, 16),  # ragged: one, several and many parts
@@ -118,3 +121,110 @@ def test_infinite_values(dev, prior, lq):
     assert (got[..., 7] == 0x7F80).all() and (got[..., 250] == 0xFF80).all()
     rest = [d for d in range(D) if d not in (7, 250)]
     assert_close(got[..., rest], exp[..., rest], "finite dims")
+
+
+class _Call:
+    """A chunk of `lq` rows after `prior` keys, on the GPU, bound to its workspace."""
+
+    def __init__(self, dev, prior, lq, capacity=8192, hole=None):
+        import torch
+        gen = torch.Generator(device=dev).manual_seed(prior + lq)
+
+        def rnd(*shape):
+            return torch.randn(shape, generator=gen, device=dev, dtype=torch.bfloat16)
+        cfg = cache_config(1, 1, 64, capacity // 64, H, D, 0)
+        table = np.arange(capacity // 64, dtype=np.int32)
+        if hole is not None:
+            table[hole] = -1
+        self.c = gk.make_config(*cfg)
+        self.args = [rnd(1, lq, 16, D), rnd(1, lq, H, D), rnd(1, lq, H, D), rnd(capacity, H, D), rnd(capacity, H, D),
+                     to_dev(table, dev), torch.tensor([prior], dtype=torch.int32, device=dev)]
+        self.lq = lq
+        need = gk.flash_attention_prefill_chunk_workspace_bytes(1, lq, self.c)
+        self.ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+
+    def plain(self):
+        import torch
+        out = torch.empty_like(self.args[0])
+        gk.check(gk.flash_attention_prefill_chunk_paged_bf16(out, *self.args, self.c, 0, 1, self.lq, 1 / 16))
+        return out
+
+    def parts(self, out=None):
+        import torch
+        out = torch.full_like(self.args[0], float("nan")) if out is None else out
+        gk.check(gk.flash_attention_prefill_chunk_paged_bf16_ws(
+            out, *self.args, self.c, 0, 1, self.lq, 1 / 16, self.ws, self.ws.numel()))
+        return out
+
+    def counters_are_zero(self):
+        return not self.ws.view(-1, SLOT_BYTES)[:, :256].any().item()
+
+
+def _close(a, b, what):
+    import torch
+    assert_close(*(from_dev_bf16(x.view(torch.int16)) for x in (a, b)), what)
+
+
+def test_a_chunk_is_one_launch(dev):
+    """In parts or not, with keys to share out or not: the host cannot know,
+    and a second launch would be paid for by short chunks as well."""
+    import torch
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    for prior, lq in ((0, 64), (2000, 64), (0, 1100)):
+        call = _Call(dev, prior, lq)
+        out = call.parts()
+        torch.cuda.synchronize()
+        stream, graph, nodes = torch.cuda.Stream(), ctypes.c_void_p(), ctypes.c_size_t()
+        handle = ctypes.c_void_p(stream.cuda_stream)
+        with torch.cuda.stream(stream):
+            assert hip.hipStreamBeginCapture(handle, 2) == 0  # relaxed
+            call.parts(out)
+            assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+        assert nodes.value == 1, (prior, lq)
+        assert hip.hipGraphDestroy(graph) == 0
+
+
+@pytest.mark.parametrize("prior,lq,hole", [(1000, 33, 3), (1000, 33, 15), (200, 100, 1), (5000, 1, 70)])
+def test_parts_over_unmapped_pages(dev, prior, lq, hole):
+    """A part without a readable key (a part is one 64-key tile in the first
+    three, as a page is), among them the last cached page; one tile of three."""
+    call = _Call(dev, prior, lq, hole=hole)
+    _close(call.parts(), call.plain(), f"hole {hole}")
+    assert call.counters_are_zero()
+
+
+def test_parts_repeat_bit_for_bit_beside_other_work(dev):
+    """Who merges depends on when the workgroups run; the bits do not. Calls
+    beside matrix products that fill the GPU, and on replays of a graph."""
+    import torch
+    x = torch.randn(4096, 4096, device=dev).bfloat16()
+    other = torch.cuda.Stream()
+    for prior, lq in ((130, 64), (7401, 93), (3000, 1), (900, 300), (400, 1000)):
+        call = _Call(dev, prior, lq)
+        print(f"prior {prior} rows {lq}", flush=True)
+        first = call.parts()
+        _close(first, call.plain(), "alone")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            for _ in range(20):
+                x @ x
+        outs = [call.parts() for _ in range(25)]
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, first) for o in outs)
+        assert call.counters_are_zero()
+        out, graph = torch.empty_like(first), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            call.parts(out)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, first)
+
+
+def test_long_parts(dev):
+    """31 parts of 40 tiles and one of 9, whose workgroup waits long."""
+    call = _Call(dev, 1248 * 64, 64, capacity=1249 * 64)
+    _close(call.parts(), call.plain(), "long")
+    assert call.counters_are_zero()
