@@ -35,7 +35,10 @@
 // Waves and splits: a split of up to 64 keys is one step of four waves. Longer
 // ones run on two waves in 69 KiB of LDS, so that a CU holds two workgroups
 // and one streams while the other starts, scores or stores (24 sequences in
-// splits of 128 / 512: 93 / 82 us against 112 / 86 on four waves).
+// splits of 128 / 512: 93 / 82 us against 112 / 86 on four waves). With split
+// counters always four: they share out the sixteen heads that the last
+// workgroup folds (8193 keys in 65 splits of 128: 65 us, on two waves 90;
+// 20000 in 250 of 80: 186 / 274; 24 sequences in splits of 512: 88 / 94).
 // K and V rows are copied into the wave's own 32 KiB of LDS with
 // global_load_lds (1 KiB, one whole row, per instruction; chunk c of key k at
 // c ^ k for K and c ^ 2 (k % 8) for V, so that the operand reads are free of
@@ -592,7 +595,8 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   for (int k = 0; k < kWaves; ++k) l_run += s_l[k][h];
 
   // ---- emit: lane holds dims 16 (wave * kWaveBlocks + d) + 4 g .. + 3 of head h
-  const bool whole_row = direct || (p.counters != nullptr && live_splits == 1);
+  const bool combines = kWaves == 4 && p.counters != nullptr;  // see launch_split_d512
+  const bool whole_row = direct || (combines && live_splits == 1);
   const int64_t row = (int64_t)b * kQueryHeads + h;
   const int dim0 = wave * kWaveBlocks * 16 + 4 * g;
   if (whole_row) {
@@ -605,7 +609,7 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   } else {
     const int64_t pidx = row * p.num_splits + split;
     const float m_nat = m_run == -INFINITY ? -INFINITY : m_run * kLn2;
-    if (p.counters != nullptr) {
+    if (combines) {
       // Device-coherent (sc1) stores: the combining workgroup may run on
       // another XCD, whose L2 does not see this XCD's write-back lines.
       if (threadIdx.x < kQueryHeads) {
@@ -632,7 +636,7 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
     }
   }
   if (owns && wave == 0) store_rows(wave_uniform(s_append[0]), token_k, token_v);
-  if (whole_row || p.counters == nullptr) return;
+  if (whole_row || !combines) return;
 
   // ---- in-kernel combine by the sequence's last split workgroup, as in
   // decode_split_kernel.
@@ -663,8 +667,8 @@ hipError_t launch(const DecodeParams &p, int32_t batch_count, hipStream_t stream
 }  // namespace
 
 hipError_t launch_split_d512(const DecodeParams &p, int32_t batch_count, hipStream_t stream) {
-  return p.balanced == 0 && p.split_size <= kD512OneStep ? launch<4>(p, batch_count, stream)
-                                                          : launch<2>(p, batch_count, stream);
+  const bool four = p.counters != nullptr || (p.balanced == 0 && p.split_size <= kD512OneStep);
+  return four ? launch<4>(p, batch_count, stream) : launch<2>(p, batch_count, stream);
 }
 
 }  // namespace gemma4

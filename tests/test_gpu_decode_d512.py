@@ -14,6 +14,7 @@ import gemma_kv as gk
 from kvtest import assert_close, cache_config, fill_page_table, from_dev_bf16, randn_bf16, ring_pages, to_dev
 from oracle import oracle
 from test_gpu_decode import _run_decode
+from test_gpu_decode_prep import _close_bits
 
 pytestmark = pytest.mark.gpu
 NAN = np.uint16(0x7FC0)
@@ -190,3 +191,61 @@ def test_keys_past_the_plan_are_not_attended_to(dev):
     got = _run_decode(dev, one, q[:1], to_dev(ck, dev), to_dev(cv, dev), pt[:cfg[3]], seq[:1], 0, 0.0442, split,
                       splits)
     assert_close(got, exp[:1], "single")
+
+
+# (split size, keys held, live lengths, token positions, split counters)
+RAW_CASES = [
+    (65, [66], [66], [65], False),                      # two waves: a step and one key
+    (96, [300], [300], [299], False),
+    (160, [700], [700], [699], False),                  # the second page lookup
+    (512, [512], [512], [511], False),                  # a single split, written directly
+    (16, [4001, 17, 2900], [4001, 17, 2900], [4000, 16, 2899], False),  # cut by the lengths
+    (96, [700, 40, 16, 333], [700, 20, 0, 333], [699, 33, 4, -1], False),  # tokens outside the live keys, none
+    (64, [300, 65], [300, 65], [299, 64], True),
+    (160, [700, 90], [700, 90], [699, 89], True),       # counters: four waves, several steps
+    (333, [1000, 40, 333], [1000, 20, 333], [999, 33, -1], True),
+]
+
+
+@pytest.mark.parametrize("split,held,seq,pos,counters", RAW_CASES)
+def test_raw_projections(dev, split, held, seq, pos, counters):
+    """The fused preparation (q, the token's K and its V from the raw K) in
+    both workgroup forms, cut by the lengths or not, combined by a launch or by
+    the counters: outputs and cache rows each on their own."""
+    import torch
+    rng = np.random.default_rng(split * 31 + len(seq))
+    cfg, pt, ck0, cv0, q, splits = _case(rng, split, held, 0, 16)
+    print(f"raw split {split}x{splits} seq {seq} pos {pos} counters {counters}", flush=True)
+    batch, max_pages, half = len(seq), cfg[3], 64
+    k = randn_bf16(rng, (batch, 1, 512), scale=3.0)
+    qw, kw = (oracle.f32_to_bf16(1.0 + 0.2 * rng.standard_normal(512).astype(np.float32)) for _ in range(2))
+    cos, sin = oracle.fill_rope_tables(max(held), half, 1_000_000.0, 512)
+    exp_k, exp_v, q_used, changed = ck0.copy(), cv0.copy(), q.copy(), []
+    for b, p in enumerate(pos):
+        if p < 0:
+            continue
+        c_row, s_row = cos[p * half:(p + 1) * half], sin[p * half:(p + 1) * half]
+        for h in range(16):
+            q_used[b, h] = oracle.prep_head(q[b, h], qw, c_row, s_row, 128)
+        row = pt[b * max_pages + p // 16] * 16 + p % 16
+        exp_k[row, 0] = oracle.prep_head(k[b, 0], kw, c_row, s_row, 128)
+        exp_v[row, 0] = oracle.prep_head(k[b, 0], None, None, None, 128)
+        changed.append(row)
+    exp = oracle.decode_attention(q_used, exp_k, exp_v, pt, seq, cfg, 0, 0.0442)
+
+    n = batch * 16 * splits
+    pm, pl, pa = (torch.full((n * d,), float("nan"), device=dev) for d in (1, 1, 512))
+    cnt = torch.zeros(batch, dtype=torch.int32, device=dev) if counters else None
+    ck, cv, out = to_dev(ck0, dev), to_dev(cv0, dev), to_dev(np.full_like(q, NAN), dev)
+    gk.check(gk.flash_attention_prep_append_decode_paged_bf16(
+        out, pm, pl, pa, to_dev(q, dev), ck, cv, to_dev(pt, dev), to_dev(np.int32(seq), dev),
+        to_dev(np.int32(pos), dev), to_dev(k, dev), None, to_dev(qw, dev), to_dev(kw, dev), to_dev(cos, dev),
+        to_dev(sin, dev), gk.make_config(*cfg), 0, 0.0442, split, splits, batch, split_counters=cnt))
+    torch.cuda.synchronize()
+    assert not counters or not cnt.any().item()
+    got_k, got_v = (from_dev_bf16(x).reshape(ck0.shape) for x in (ck, cv))
+    rest = np.setdiff1d(np.arange(len(ck0)), changed)
+    assert np.array_equal(got_k[rest], ck0[rest]) and np.array_equal(got_v[rest], cv0[rest])
+    _close_bits(got_k[changed], exp_k[changed], "cache K")
+    _close_bits(got_v[changed], exp_v[changed], "cache V")
+    assert_close(from_dev_bf16(out).reshape(exp.shape), exp, "attention")
