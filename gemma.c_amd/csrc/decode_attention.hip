@@ -241,7 +241,7 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
     store128(p.cache_v + dst, load128(p.new_v + src));
   };
 
-  if (key_count == 0 && direct) {
+  if (key_count == 0 && split == 0 && (direct || p.counters != nullptr)) {
     // No live key: the row is defined as zeros (src/...decode.cu:733-743).
     if (key_lane == 0 && r == 0) {
 #pragma unroll

@@ -202,6 +202,7 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   const int32_t key_count = min(seq_len > first ? seq_len - first : 0, capacity);
   const int32_t live_splits = (key_count + split_size - 1) / split_size;
   const bool direct = p.num_splits == 1;
+  const bool combines = kWaves == 4 && p.counters != nullptr;  // see launch_split_d512
 
   if (p.gate != nullptr && wave_uniform(gate_word) != 0) {
     // A failed step: no append; a direct launch zeroes its rows (the combine
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   };
 
   if (split >= live_splits) {
-    if (key_count == 0 && direct) {
+    if (key_count == 0 && split == 0 && (direct || combines)) {
       // No live key: the row is defined as zeros (src/...decode.cu:733-743).
       uint16_t *rows = p.out + (int64_t)b * kQueryHeads * kDim;
       for (int e = threadIdx.x; e < kQueryHeads * kRowChunks; e += kWaves * kWave)
@@ -595,7 +596,6 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   for (int k = 0; k < kWaves; ++k) l_run += s_l[k][h];
 
   // ---- emit: lane holds dims 16 (wave * kWaveBlocks + d) + 4 g .. + 3 of head h
-  const bool combines = kWaves == 4 && p.counters != nullptr;  // see launch_split_d512
   const bool whole_row = direct || (combines && live_splits == 1);
   const int64_t row = (int64_t)b * kQueryHeads + h;
   const int dim0 = wave * kWaveBlocks * 16 + 4 * g;

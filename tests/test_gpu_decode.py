@@ -487,3 +487,33 @@ def test_decode_randomized_against_oracle(dev, seed):
     for b, n in enumerate(seq):
         if n == 0:
             assert not got[b].any(), what
+
+
+@pytest.mark.parametrize("heads,dim,split", [(8, 256, 32), (1, 512, 64), (1, 512, 96)])
+def test_empty_sequence_with_split_counters(dev, heads, dim, split):
+    """A sequence without live keys has no split workgroup that would combine:
+    its rows are zeros all the same, and its token is appended."""
+    import torch
+    rng = np.random.default_rng(dim + split)
+    held, seq, pos = [200, 16, 70], [200, 0, 70], [199, 4, 69]
+    cfg = cache_config(1, 3, 16, 13, heads, dim, 0)
+    pt = fill_page_table(cfg, held)
+    ck0, cv0 = (randn_bf16(rng, (3 * 13 * 16, heads, dim)) for _ in range(2))
+    q, k, v = (randn_bf16(rng, (3, h, dim)) for h in (16, heads, heads))
+    exp_k, exp_v = ck0.copy(), cv0.copy()
+    oracle.kv_cache_write(exp_k, exp_v, cfg, pt, [0, 1, 2], pos, 0, k, v)
+    exp = oracle.decode_attention(q, exp_k, exp_v, pt, seq, cfg, 0, 0.05)
+    counters = torch.zeros(3 * heads, dtype=torch.int32, device=dev)
+    out = to_dev(np.full_like(q, 0x7FC0), dev)
+    n = 3 * 16 * -(-200 // split)
+    pm, pl, pa = (torch.full((n * d,), float("nan"), device=dev) for d in (1, 1, dim))
+    ck, cv = to_dev(ck0, dev), to_dev(cv0, dev)
+    gk.check(gk.flash_attention_append_decode_paged_bf16(
+        out, pm, pl, pa, to_dev(q, dev), ck, cv, to_dev(pt, dev), to_dev(np.int32(seq), dev),
+        to_dev(np.int32(pos), dev), to_dev(k, dev), to_dev(v, dev), gk.make_config(*cfg), 0, 0.05, split,
+        -(-200 // split), 3, split_counters=counters))
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev_bf16(ck).reshape(exp_k.shape), exp_k)
+    assert np.array_equal(from_dev_bf16(cv).reshape(exp_v.shape), exp_v)
+    assert_close(from_dev_bf16(out).reshape(exp.shape), exp, "empty sequence")
+    assert not counters.any().item()
