@@ -653,7 +653,7 @@ template <int kDim>
 constexpr int combine_dims() { return kDim == 512 ? 32 : 64; }
 
 template <int kDim, bool kBalanced, int kCombineDims = combine_dims<kDim>()>
-__global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(DecodeParams p) {
+__global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(CombineParams p) {
   constexpr int kCombineLanes = kCombineThreads / (kCombineDims / 4);  // split lanes
   constexpr int kGroups = kCombineDims / 4;      // 4-dim groups: threads per split lane
   constexpr int kWaves = kCombineThreads / kWave;
@@ -714,7 +714,7 @@ __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(DecodeP
     int32_t seq_len = seq_word;
     asm volatile("" : "+v"(seq_len));
     seq_len = wave_uniform(seq_len);
-    int32_t first = p.c.window_size > 0 ? seq_len - p.c.window_size : 0;
+    int32_t first = p.window_size > 0 ? seq_len - p.window_size : 0;
     first = first < 0 ? 0 : first;
     const int32_t key_count = seq_len > first ? seq_len - first : 0;
     const int32_t splits =
@@ -829,7 +829,7 @@ hipError_t launch_split_256(const DecodeParams &p, int32_t batch_count, hipStrea
 }
 
 template <int kDim>
-hipError_t launch_combine(const DecodeParams &p, int32_t batch_count, hipStream_t stream) {
+hipError_t launch_combine(const CombineParams &p, int32_t batch_count, hipStream_t stream) {
   auto launch = [&](auto *kernel, int dims) {
     hipLaunchKernelGGL(kernel, dim3(batch_count * kQueryHeads, kDim / dims), dim3(kCombineThreads),
                        0, stream, p);
@@ -912,8 +912,11 @@ hipError_t decode_entry(uint16_t *out, float *pm, float *pl, float *pacc,
   const hipError_t e = d512 ? launch_split_d512(p, batch_count, stream)
                             : launch_split_256(p, batch_count, stream);
   if (e != hipSuccess || !combine || num_splits == 1 || p.counters != nullptr) return e;
-  return d512 ? launch_combine<512>(p, batch_count, stream)
-              : launch_combine<256>(p, batch_count, stream);
+  const CombineParams cp = {p.out,         p.partial_m,  p.partial_l,  p.partial_acc,
+                            p.seq_lengths, p.gate,       c.window_size, p.split_size,
+                            p.num_splits,  p.balanced,   p.batch};
+  return d512 ? launch_combine<512>(cp, batch_count, stream)
+              : launch_combine<256>(cp, batch_count, stream);
 }
 
 constexpr int kMaxDevices = 64;
@@ -1093,13 +1096,13 @@ hipError_t gemma4_flash_attention_decode_combine_bf16(
       d_partial_l == nullptr || d_partial_acc == nullptr || d_seq_lengths == nullptr) {
     return hipErrorInvalidValue;
   }
-  DecodeParams p{};
+  CombineParams p{};
   p.out = reinterpret_cast<uint16_t *>(d_out);
-  p.partial_m = const_cast<float *>(d_partial_m);
-  p.partial_l = const_cast<float *>(d_partial_l);
-  p.partial_acc = const_cast<float *>(d_partial_acc);
+  p.partial_m = d_partial_m;
+  p.partial_l = d_partial_l;
+  p.partial_acc = d_partial_acc;
   p.seq_lengths = d_seq_lengths;
-  p.c.window_size = config.window_size;
+  p.window_size = config.window_size;
   p.split_size = split_size;
   p.num_splits = num_splits;
   if (config.head_dim == 256) return launch_combine<256>(p, batch_count, stream);

@@ -46,6 +46,25 @@ struct DecodeParams {
   int32_t batch = 0;
 };
 
+// Arguments of the combine kernel: what it reads and no more. A launch's
+// arguments come cold from memory (2048 decode steps with their own arguments
+// each, as a graph: 8.49 us a step with the whole DecodeParams, 8.28 so).
+struct CombineParams {
+  uint16_t *out;
+  const float *partial_m;
+  const float *partial_l;
+  const float *partial_acc;
+  const int32_t *seq_lengths;
+  const int32_t *gate;
+  int32_t window_size;
+  int32_t split_size;
+  int32_t num_splits;
+  int32_t balanced;
+  int32_t batch;
+};
+__device__ __forceinline__ int32_t window_of(const DecodeParams &p) { return p.c.window_size; }
+__device__ __forceinline__ int32_t window_of(const CombineParams &p) { return p.window_size; }
+
 constexpr int kRowInvalid = -1;   // key outside the split or unmapped page
 constexpr int kRowNewToken = -2;  // key being appended in this launch
 
@@ -224,7 +243,8 @@ struct BalancedCut {
   int32_t size;    // keys per split
   int32_t splits;  // of this lane's sequence (0 past the batch)
 };
-__device__ __forceinline__ BalancedCut balanced_cut(const DecodeParams &p, int32_t keys) {
+template <class Params>
+__device__ __forceinline__ BalancedCut balanced_cut(const Params &p, int32_t keys) {
   const int lane = __lane_id();
   // The plan's slots bound what a sequence can hold, as with fixed splits.
   const int64_t capacity = (int64_t)p.split_size * p.num_splits;
@@ -256,13 +276,13 @@ __device__ __forceinline__ BalancedCut balanced_cut(const DecodeParams &p, int32
   return cut;
 }
 // Live keys of sequence `lane` of the batch (0 past it).
-__device__ __forceinline__ int32_t lane_live_keys(const DecodeParams &p) {
+template <class Params>
+__device__ __forceinline__ int32_t lane_live_keys(const Params &p) {
   const int lane = __lane_id();
   const int32_t len = p.seq_lengths[lane < p.batch ? lane : 0];
-  const int32_t first = p.c.window_size > 0 ? max(len - p.c.window_size, 0) : 0;
+  const int32_t first = window_of(p) > 0 ? max(len - window_of(p), 0) : 0;
   return lane < p.batch && len > first ? len - first : 0;
 }
-
 
 // Split phase of the 1 x 512 geometry (decode_d512.hip) on a grid of
 // (p.num_splits, batch_count); checked arguments.
