@@ -1147,12 +1147,16 @@ hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
   // 13.0 / 12.6 / 12.4 us). A batch takes single steps where they fit one
   // round of the chip (8 of 100-1000 keys 12 us, 31 in splits of 16 on the
   // former kernel), and kD512BatchSplit keys at least otherwise: the launch
-  // then sizes them by the lengths (balanced_cut).
+  // then sizes them by the lengths (balanced_cut). The count never drops from
+  // the one to the other (it would be 128, then 86 for two sequences of 8192 /
+  // 8193 keys): partials sized for the longest length hold shorter plans'.
+  int64_t fewest = 1;
   if (planned && config.head_dim == 512) {
     const int64_t steps = (keys + kD512OneStep - 1) / kD512OneStep;
     if (steps == 1 || (batch_count > 1 && steps * batch_count <= kD512Cus)) {
       size = kD512OneStep;
     } else {
+      if (batch_count > 1) fewest = std::max<int64_t>(kD512Cus / batch_count, 1);
       size = std::max<int64_t>(size, batch_count > 1 ? kD512BatchSplit : kD512OneStep - tile);
     }
   }
@@ -1166,7 +1170,7 @@ hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
     size = key_tile;
   }
   *split_size = (int32_t)size;
-  *num_splits = (int32_t)((keys + size - 1) / size);
+  *num_splits = (int32_t)std::max((keys + size - 1) / size, fewest);
   return hipSuccess;
 }
 

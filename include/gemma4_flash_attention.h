@@ -209,15 +209,20 @@ hipError_t gemma4_flash_attention_global_fwd_bf16_norm_rope(
     int seqlen_k, float softmax_scale, hipStream_t stream);
 
 // Split plan for the MI355X: the split size (a multiple of the kernel's key
-// wave chunk) that gives about `target_workgroups` split workgroups (0 = default:
-// one per CU for one sequence, 32 per CU for a batch) for `batch_count`
-// sequences of up to `max_live_keys` live keys, and the split count that covers `max_live_keys`. With the default target,
-// one sequence whose splits would hold two key tiles or fewer (a 1024-key
-// sliding window) gets one-tile splits instead, up to two workgroups per CU;
-// a batch's splits at 1 x 512 hold 96 keys at least (its combining launches
-// lengthen them by the lengths on the device). Replaces the fixed
-// GEMMA4_SLIDING_DECODE_SPLIT_SIZE (src/gemma4.h:24) and the active split
-// count of src/gemma4_decode_megakernel.cu:158-167.
+// wave chunk) that gives about `target_workgroups` split workgroups (0 =
+// default: one per CU for one sequence, 32 per CU for a batch) for
+// `batch_count` sequences of up to `max_live_keys` live keys, and a split
+// count that covers `max_live_keys`. With the default target, one sequence
+// whose splits would hold two key tiles or fewer (a 1024-key sliding window)
+// gets one-tile splits instead, up to two workgroups per CU; splits at 1 x 512
+// hold 48 keys at least, a batch's 64 (while one round of the chip takes them
+// all) or 96, and launches that combine a batch size them anew by the lengths
+// on the device, shorter or longer.
+// The count is not monotonic in `max_live_keys`: where the split size steps up
+// it drops. Size the partials for the plan that is passed; a plan made for the
+// longest length may be passed for every shorter one.
+// Replaces the fixed GEMMA4_SLIDING_DECODE_SPLIT_SIZE (src/gemma4.h:24) and
+// the active split count of src/gemma4_decode_megakernel.cu:158-167.
 hipError_t gemma4_decode_split_plan(Gemma4KvCacheConfig config,
                                     int32_t batch_count, int32_t max_live_keys,
                                     int32_t target_workgroups,

@@ -102,3 +102,15 @@ def test_split_plan_fills_the_chip():
     # 1 x 512 (staged 16-key steps): 8193 keys as 171 splits of 48.
     c = gk.make_config(8, 129, 64, 129, 1, 1, 512, 0)
     assert gk.decode_split_plan(c, 1, 8193) == (48, 171)
+
+
+@pytest.mark.parametrize("batch", [2, 3, 8, 24, 64])
+def test_split_plan_1x512_batch_slots_do_not_drop(batch):
+    """From one-step splits to longer ones a batch's slot count never drops:
+    partials sized for the longest length hold every shorter plan's."""
+    c = gk.make_config(1, batch * 512, 64, 512, batch, 1, 512, 0)
+    most = 0
+    for keys in range(1, min(96 * (8192 // batch), 20000) + 1):
+        size, n = gk.decode_split_plan(c, batch, keys)
+        assert size in (64, 96) and size * n >= keys and n >= most, (keys, size, n, most)
+        most = n
