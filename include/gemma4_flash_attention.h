@@ -26,13 +26,16 @@ extern "C" {
 //                  [max(0, len - window_size), len) for a sliding cache and
 //                  [0, len) for a global one
 //   d_page_table   [batch_size][max_pages_per_seq] physical page per ring slot
-//   partials       partial_m/l [(row * num_splits + split)],
-//                  partial_acc [(row * num_splits + split) * head_dim + d],
-//                  row = b * 16 + q_head. Unused when num_splits == 1 (the
-//                  single split writes d_out directly; may then be null).
-// Split `s` covers live keys [first + s*split_size, first + (s+1)*split_size);
-// splits past the live count do nothing. Supported geometries:
-// (num_heads, head_dim) = (8, 256) and (1, 512); 16 query heads.
+//   partials       scratch of batch_count * 16 * num_splits floats (partial_m,
+//                  partial_l) and head_dim times as many (partial_acc). What
+//                  is in it afterwards is not defined: the splits may be cut
+//                  by ring slot or by the lengths instead of by split_size
+//                  (only gemma4_flash_attention_decode_split_paged_bf16
+//                  leaves partials to combine). Unused when num_splits == 1
+//                  (the single split writes d_out directly; may then be null).
+// The splits cover split_size * num_splits live keys from the first on; more
+// are not attended to. Supported geometries: (num_heads, head_dim) = (8, 256)
+// and (1, 512); 16 query heads.
 hipError_t gemma4_flash_attention_decode_paged_bf16(
     gemma4_bf16 *d_out, float *d_partial_m, float *d_partial_l,
     float *d_partial_acc, const gemma4_bf16 *d_q, const gemma4_bf16 *d_cache_k,
@@ -114,7 +117,11 @@ hipError_t gemma4_flash_attention_prep_append_decode_paged_bf16(
 // phase (phase_decode_paged_grouped_split,
 // src/gemma4_flash_attention_decode.cu:691-878), with the fused append of
 // gemma4_flash_attention_append_decode_paged_bf16 when d_token_position is not
-// null; with num_splits == 1 it writes d_out directly. The combine phase
+// null; with num_splits == 1 it writes d_out directly. Its partials are
+// partial_m/l [row * num_splits + split] and partial_acc [(row * num_splits +
+// split) * head_dim + d], row = b * 16 + q_head, where split s covers live keys
+// [first + s*split_size, first + (s+1)*split_size); splits past the live count
+// are not written. The combine phase
 // (phase_decode_paged_reduce, src/gemma4_flash_attention_decode.cu:880-977)
 // reduces the live splits of every (batch, query head) row into d_out.
 hipError_t gemma4_flash_attention_decode_split_paged_bf16(
