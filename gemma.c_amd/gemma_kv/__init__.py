@@ -167,8 +167,13 @@ def _current_stream() -> int:
     if _raw_stream is None:
         import torch
         handle = torch.cuda.current_stream().cuda_stream  # initialises torch's runtime
-        get, device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
-        _raw_stream = lambda: get(device())  # noqa: E731  (0.2 us; a Stream object takes 2.9)
+        # Names of torch's own that it may drop: the public call stays the fallback.
+        get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        device = getattr(torch._C, "_cuda_getDevice", None)
+        if get is not None and device is not None:
+            _raw_stream = lambda: get(device())  # noqa: E731  (0.2 us; a Stream object takes 2.9)
+        else:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
         return handle
     return _raw_stream()
 

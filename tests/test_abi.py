@@ -114,3 +114,22 @@ def test_split_plan_1x512_batch_slots_do_not_drop(batch):
         size, n = gk.decode_split_plan(c, batch, keys)
         assert size in (64, 96) and size * n >= keys and n >= most, (keys, size, n, most)
         most = n
+
+
+@pytest.mark.parametrize("missing", [(), ("_cuda_getCurrentRawStream",), ("_cuda_getDevice",)])
+def test_stream_handle_needs_no_torch_internals(monkeypatch, missing):
+    """The current stream is looked up on every call, through torch's raw
+    lookup where it has one and through the public call otherwise."""
+    import types
+
+    import torch
+    current = [7]
+    monkeypatch.setattr(gk, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=current[0]))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 3, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda d: current[0] if d == 3 else None, raising=False)
+    for name in missing:
+        monkeypatch.delattr(torch._C, name)
+    for handle in (7, 8, 9):
+        current[0] = handle
+        assert gk.stream_handle() == handle
