@@ -108,8 +108,10 @@ __global__ __launch_bounds__(kRowWaves *kWave) void o_projection_rows_kernel(
 // 4096, 8 rows 12.9 -> 11.6, 64 25.1 -> 15.5, 128 39.8 -> 18.9. With four
 // copies of the weights in turn, which the 256 MiB Infinity Cache still helps:
 // width 8192, 24 rows 30.5 -> 15.1 (kernel 26.2 -> 13.0), 256 155 -> 37.
-// Nontemporal weight copies gain 1-2 us from HBM up to 24 rows (8192, 8 rows
-// 17.1) but give up that help (24 rows 19.0 against 15.1), and lose from 64 rows on.
+// Not taken: nontemporal weight copies. From HBM they gain 1-2 us up to 24
+// rows (8192, 8 rows 17.1) and lose from 64 rows on; with weights that the
+// Infinity Cache holds they lose 4 (24 rows 19.0 against 15.1). (The GEMV for
+// few rows gains from HBM and loses nothing there.)
 constexpr int kSplit = 4;  // waves per workgroup, one k slice each
 constexpr int kChunkK = 64;
 constexpr int kBlockUint4 = 16 * kChunkK / kPackElems;  // 16 rows of a chunk: 2 KiB
@@ -304,7 +306,11 @@ template <int kWidth>
 hipError_t launch_projection(const uint16_t *attn, const uint16_t *w, uint16_t *residual,
                              int32_t rows, hipStream_t stream) {
   using S = RowShape<kWidth>;
-  if (rows <= S::kFewRows) {
+  // The MFMA kernel's copies into LDS take 16-byte aligned chunks; the GEMV's
+  // loads may start anywhere.
+  const bool aligned =
+      ((reinterpret_cast<uintptr_t>(attn) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+  if (rows <= S::kFewRows || !aligned) {
     hipLaunchKernelGGL(o_projection_rows_kernel<kWidth>, dim3(S::kGroups), dim3(kRowWaves * kWave),
                        0, stream, attn, w, residual, rows);
     return hipGetLastError();

@@ -128,3 +128,25 @@ def test_o_projection_block_edges(dev, rows, width):
     scale = outs[0].double().square().mean(-1, keepdim=True).add(1e-6).rsqrt()
     assert torch.allclose(outs[1].double(), outs[0].double() * scale, rtol=2.0 ** -7, atol=1e-6)
     assert torch.equal(outs[2], outs[1])
+
+
+@pytest.mark.parametrize("rows,width,off_a,off_w", [(5, 4096, 1, 0), (9, 8192, 0, 3), (33, 4096, 4, 8), (8, 4096, 8, 0)])
+def test_o_projection_unaligned_operands(dev, rows, width, off_a, off_w):
+    """Attention rows and weights that start off 16 bytes (offsets in elements;
+    8 is aligned): the same result as from aligned copies up to the order of
+    the sum."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows)
+
+    def at(offset, *shape):
+        flat = torch.randn(shape[0] * shape[1] + offset, generator=gen, device=dev).bfloat16()
+        return flat[offset:].view(shape)
+    a, w = at(off_a, rows, width), at(off_w, HIDDEN, width)
+    assert (a.data_ptr() % 16 == 0) == (off_a % 8 == 0)
+    g = torch.ones(HIDDEN, device=dev).bfloat16()
+    x = torch.zeros((rows, HIDDEN), device=dev).bfloat16()
+    outs = [torch.full((rows, HIDDEN), float("nan"), device=dev).bfloat16() for _ in range(3)]
+    gk.check(gk.attention_o_projection_post_norm_bf16(*outs, a, w, g, x, rows, width))
+    exact = a.double() @ w.double().T
+    bound = exact.abs() * 2.0 ** -8 + (a.double().abs() @ w.double().abs().T) * 2.0 ** -24 * 16
+    assert bool(((outs[0].double() - exact).abs() <= bound).all())
