@@ -86,9 +86,7 @@ struct DecodeShape {
   static constexpr int S = __builtin_ctz(LPR / NP);       // duplicate-lane bits
   static constexpr int GB = __builtin_ctz(GW);            // head-select bits
   static constexpr int kRowElems = kHeads * kDim;
-  // Rotary dims of the geometry: all of a sliding head, a quarter of a
-  // global one (src/gemma4.h rotary settings).
-  static constexpr int kRot = kHeads == 1 ? kDim / 4 : kDim;
+  static constexpr int kRot = kDim;  // rotary dims: the whole head
   static constexpr int kMaxW = kWaves;  // waves of a split workgroup at most
   static_assert(G % GW == 0, "heads per wave must divide the GQA group");
   static_assert(NP <= LPR, "one reduced score per lane at most");
@@ -212,9 +210,8 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
         const float *sin_row = p.sin + (int64_t)new_pos * (Sh::kRot / 2);
         const uint4 raw_k = load128(p.new_k + src);
         const uint4 kp = prep_pack<LPR, Sh::kRot>(raw_k, p.k_norm_weight, cos_row, sin_row, cpack);
-        // The 1x512 geometry derives V from the raw K (no V projection).
-        const uint4 raw_v = p.new_v != nullptr ? load128(p.new_v + src) : raw_k;
-        const uint4 vp = prep_pack<LPR, Sh::kRot>(raw_v, nullptr, cos_row, sin_row, cpack);
+        const uint4 vp = prep_pack<LPR, Sh::kRot>(load128(p.new_v + src), nullptr, cos_row,
+                                                  sin_row, cpack);
         if (r == 0) {
           const int64_t dst = (int64_t)new_row * Sh::kRowElems + (int64_t)head * D +
                               cpack * kPackElems;
@@ -645,8 +642,8 @@ constexpr int kCombineThreads = 256;
 // A batch cut by its lengths (kBalanced) reads its live slots only; over four
 // sequences, 128 dims per workgroup (24 sequences: 6.9 against 26 us with 32,
 // whose 6144 workgroups each derive the cut).
-// Dims per workgroup otherwise: 64 for 256-dim rows (16 split lanes), 32 for 512-dim
-// rows (32 split lanes: the 1 x 512 layer's ~129 splits fold in shorter
+// Dims per workgroup otherwise: 64 for 256-dim rows (16 split lanes), 32 for
+// 512-dim rows (32 split lanes: the 1 x 512 layer's splits fold in shorter
 // chains; 24.0 against 24.8 us per layer, while 32 dims for 256-dim rows
 // measured ~1% slower on the per-layer and batch-64 legs).
 template <int kDim>
@@ -901,8 +898,9 @@ hipError_t decode_entry(uint16_t *out, float *pm, float *pl, float *pacc,
   // A batch whose combine follows is cut by its lengths (balanced_cut): two
   // workgroups per CU, all resident at once. Not one that takes a single
   // round of one-step workgroups as planned (2 x 500-1000 keys: 12.4 against
-  // 17 us). One sequence is planned by its length already, except in a step (gate), which plans by the cache's
-  // capacity: a cut there once that gives splits of more than one step.
+  // 17 us). One sequence is planned by its length already, except in a step
+  // (gate), which plans by the cache's capacity: a cut there once that gives
+  // splits of more than one step.
   const bool one_round = split_size <= kD512OneStep && (int64_t)num_splits * batch_count <= kD512Cus;
   if (d512 && combine && p.counters == nullptr && num_splits > 1 && batch_count <= kBalancedBatch &&
       (batch_count >= 2 ? !one_round : (gate != nullptr && split_size > kD512OneStep))) {

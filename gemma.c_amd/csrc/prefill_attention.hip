@@ -925,7 +925,8 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
       }
     }
   }
-  if constexpr (kMode == Mode::kPaired) __syncthreads();  // the next unit reuses the LDS stages and tables
+  // The next unit reuses the LDS stages and tables.
+  if constexpr (kMode == Mode::kPaired) __syncthreads();
   }  // units
   if constexpr (kMode == Mode::kParts) {
     if (live_parts > 1) merge_parts(p, b, part_blk, head, part, live_parts, per_part, &s_shares);
