@@ -120,12 +120,6 @@ __device__ __forceinline__ float *part_partial(char *ws, int64_t i) {
   return reinterpret_cast<float *>(ws + (i >> 1) * kSlotBytes + kSlotCounterBytes +
                                    (i & 1) * kPartialBytes);
 }
-// A row block's share of `tiles` key tiles in parts: tiles per part. One tile
-// is worth a workgroup of its own (64 rows after 37 keys, two tiles: in one
-// part 13.6 us, in two 11.6).
-__device__ __forceinline__ int part_tiles(int tiles, int n_parts) {
-  return tiles <= n_parts ? 1 : (tiles + n_parts - 1) / n_parts;
-}
 // Key tiles of causal row block blk (no window).
 __device__ __forceinline__ int causal_tiles(int prior, int chunk_len, int blk) {
   return (prior + min(kPrefillRows * (blk + 1), chunk_len) - 1) / kTileKeys + 1;
@@ -143,6 +137,26 @@ __device__ __forceinline__ int div_small(int n, int d, float inv_d) {
   q += (q + 1) * d <= n ? 1 : 0;
   q -= q * d > n ? 1 : 0;
   return q;
+}
+
+// Tiles per part at most, of a chunk in parts: one number for the row blocks of
+// a sequence, whose workgroups run at once, so that the last block sets the
+// time. A row block's partial of 64 rows is written and read once, 266 KB, and
+// takes the launch 1 / kPartialsPerTile of a tile's 1.9 us. With `load` = rows x
+// KV heads of the batch and mean = (first + last) / 2 tiles per block, per +
+// load / 64 * mean / per / kPartialsPerTile tiles of time are least at the
+// square root below. No block is shared out where that saves less than it costs.
+// As many parts as there are workgroups, and so: 16 x 64 rows after 64 keys in a
+// cache of 4096 22.3 -> 14.8 us (plain form 14.5), 8 x 128 after 100 22.6 -> 18.3
+// (balanced pairs 18.4), 3 x 64 after 896 20.7 -> 20.1 (plain 37.5).
+constexpr int kPartialsPerTile = 53;
+__device__ __forceinline__ int part_tiles(int first, int last, int n_parts, int load) {
+  constexpr float kUnit = 2.0f * kPrefillRows * kPartialsPerTile;
+  const float cost = (float)load * (float)(first + last);
+  int per = max((int)(__builtin_amdgcn_sqrtf(cost * (1.0f / kUnit)) + 0.5f), 1);
+  if (per * n_parts < last) per = (last + n_parts - 1) / n_parts;
+  const int parts = div_small(last + per - 1, per, __builtin_amdgcn_rcpf((float)per));
+  return (float)(last - per) * (float)last * kUnit > cost * (float)parts ? per : last;
 }
 
 typedef unsigned u32x4v_t __attribute__((ext_vector_type(4)));
@@ -306,9 +320,9 @@ __device__ __forceinline__ void merge_columns(char *ws, int64_t part0, int live_
 // not depend on who merges.
 // A second launch for the merge, as before, was paid for by every chunk, also
 // if its row blocks are one part each: the device knows that, the host does
-// not. 64 rows after 0 / 37 / 300 keys in a cache of 8192: 12.8 / 15.1 / 13.9
-// -> 11.3 / 11.6 / 13.0 us (plain form 11.05 / 13.1 / 20.9); 93 rows after 7401
-// 32.9 -> 31.6. The workgroups without keys matter: merged by the others alone
+// not. 64 rows after 0 / 64 / 320 keys in a cache of 4096: 12.8 / 14.9 / 13.8
+// -> 11.2 / 11.6 / 13.1 us (plain form 11.1 / 12.9 / 20.7); 93 rows after 7401
+// 33.7 -> 31.8. The workgroups without keys matter: merged by the others alone
 // 64 rows after 300 took 16.5. So does little code, which runs once, cold:
 // eight columns and four parts unrolled, 18.4.
 constexpr uint64_t kMergeWaitTicks = 200;  // per tile of a part: 2 us at 100 MHz
@@ -424,20 +438,30 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   Unit unit0 = {0, 0, 0, -1, 0}, unit1 = {0, 0, 0, -1, 0};
   int n_units = 0;
   int part = 0, live_parts = 1, part_blk = 0, per_part = 0;
+  int part_lo = 0, part_hi = kAllTiles;
+  auto settle_part = [&]() __attribute__((always_inline)) {
+    const int tiles = causal_tiles(prior, Lq, part_blk);
+    per_part = wave_uniform(part_tiles(causal_tiles(prior, Lq, 0), (prior + Lq - 1) / kTileKeys + 1,
+                                       p.n_parts, gridDim.y * Lq * Hk));
+    live_parts = wave_uniform(
+        div_small(tiles + per_part - 1, per_part, __builtin_amdgcn_rcpf((float)per_part)));
+    // An even share of the tiles.
+    const float inv = __builtin_amdgcn_rcpf((float)live_parts);
+    part_lo = wave_uniform(div_small(tiles * part, live_parts, inv));
+    part_hi = part == live_parts - 1
+                  ? kAllTiles : wave_uniform(div_small(tiles * (part + 1), live_parts, inv));
+  };
   if constexpr (kMode == Mode::kParts) {
     // Grid z is the part: the first parts, often the only ones, start first.
     part = blockIdx.z;
     part_blk = blockIdx.x / Hk;
-    const int tiles = causal_tiles(prior, Lq, part_blk);
-    per_part = part_tiles(tiles, p.n_parts);
-    live_parts = per_part == 1 ? tiles : (tiles + per_part - 1) / per_part;
-    if (part < live_parts) {
-      unit0 = {kPrefillRows * part_blk, part * per_part,
-               part == live_parts - 1 ? kAllTiles : (part + 1) * per_part, -1, 0};
-      n_units = 1;
-    } else if (live_parts == 1) {
-      return;
-    }
+    unit0 = {kPrefillRows * part_blk, 0, kAllTiles, -1, 0};
+    // Part 0 has keys whatever the length is, and settles its share while its
+    // query rows are on the way (64 rows without prior, two sequences: 11.5 us
+    // ahead of those loads, 11.2 so).
+    if (part != 0) settle_part();
+    n_units = part < live_parts ? 1 : 0;
+    if (n_units == 0 && live_parts == 1) return;
   } else if constexpr (kMode == Mode::kPaired) {
     const int rest = blockIdx.x / Hk;
     const int pair = rest >> 1, side = rest & 1;
@@ -476,8 +500,8 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
   for (int u = 0; u < n_units; ++u) {
   const Unit &cur = u == 0 ? unit0 : unit1;
   const int q0 = wave_uniform(cur.q0);
-  const int unit_lo = wave_uniform(cur.t_lo);
-  const int unit_hi = wave_uniform(cur.t_hi);
+  int unit_lo = wave_uniform(cur.t_lo);
+  int unit_hi = wave_uniform(cur.t_hi);
   const int unit_slot = wave_uniform(cur.slot);
   const int unit_part = wave_uniform(cur.part);
 
@@ -507,6 +531,11 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void prefill_chunk_kernel(Prefi
       const uint4 x = row_ok ? load128(qrow + 16 * s + 8 * half) : make_uint4(0, 0, 0, 0);
       qreg[s] = u32x4v_t{x.x, x.y, x.z, x.w};
     }
+  }
+  if constexpr (kMode == Mode::kParts) {
+    if (part == 0) settle_part();
+    unit_lo = part_lo;
+    unit_hi = part_hi;
   }
 
   // Key range of the workgroup (absolute positions), tile-aligned start.

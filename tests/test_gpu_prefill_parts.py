@@ -124,36 +124,37 @@ def test_infinite_values(dev, prior, lq):
 
 
 class _Call:
-    """A chunk of `lq` rows after `prior` keys, on the GPU, bound to its workspace."""
+    """A chunk of `lq` rows after `prior` keys for each sequence, on the GPU, bound to its workspace."""
 
-    def __init__(self, dev, prior, lq, capacity=8192, hole=None):
+    def __init__(self, dev, prior, lq, capacity=8192, hole=None, batch=1):
         import torch
         gen = torch.Generator(device=dev).manual_seed(prior + lq)
 
         def rnd(*shape):
             return torch.randn(shape, generator=gen, device=dev, dtype=torch.bfloat16)
-        cfg = cache_config(1, 1, 64, capacity // 64, H, D, 0)
-        table = np.arange(capacity // 64, dtype=np.int32)
+        cfg = cache_config(1, batch, 64, capacity // 64, H, D, 0)
+        table = np.arange(batch * (capacity // 64), dtype=np.int32)
         if hole is not None:
             table[hole] = -1
         self.c = gk.make_config(*cfg)
-        self.args = [rnd(1, lq, 16, D), rnd(1, lq, H, D), rnd(1, lq, H, D), rnd(capacity, H, D), rnd(capacity, H, D),
-                     to_dev(table, dev), torch.tensor([prior], dtype=torch.int32, device=dev)]
-        self.lq = lq
-        need = gk.flash_attention_prefill_chunk_workspace_bytes(1, lq, self.c)
+        rows = batch * capacity
+        self.args = [rnd(batch, lq, 16, D), rnd(batch, lq, H, D), rnd(batch, lq, H, D), rnd(rows, H, D), rnd(rows, H, D),
+                     to_dev(table, dev), torch.tensor([prior] * batch, dtype=torch.int32, device=dev)]
+        self.batch, self.lq = batch, lq
+        need = gk.flash_attention_prefill_chunk_workspace_bytes(batch, lq, self.c)
         self.ws = torch.zeros(need, dtype=torch.uint8, device=dev)
 
     def plain(self):
         import torch
         out = torch.empty_like(self.args[0])
-        gk.check(gk.flash_attention_prefill_chunk_paged_bf16(out, *self.args, self.c, 0, 1, self.lq, 1 / 16))
+        gk.check(gk.flash_attention_prefill_chunk_paged_bf16(out, *self.args, self.c, 0, self.batch, self.lq, 1 / 16))
         return out
 
     def parts(self, out=None):
         import torch
         out = torch.full_like(self.args[0], float("nan")) if out is None else out
         gk.check(gk.flash_attention_prefill_chunk_paged_bf16_ws(
-            out, *self.args, self.c, 0, 1, self.lq, 1 / 16, self.ws, self.ws.numel()))
+            out, *self.args, self.c, 0, self.batch, self.lq, 1 / 16, self.ws, self.ws.numel()))
         return out
 
     def counters_are_zero(self):
@@ -224,7 +225,25 @@ def test_parts_repeat_bit_for_bit_beside_other_work(dev):
 
 
 def test_long_parts(dev):
-    """31 parts of 40 tiles and one of 9, whose workgroup waits long."""
+    """31 parts of 39 tiles and one of 40."""
     call = _Call(dev, 1248 * 64, 64, capacity=1249 * 64)
     _close(call.parts(), call.plain(), "long")
+    assert call.counters_are_zero()
+
+
+@pytest.mark.parametrize("batch,prior,lq,shared", [
+    (1, 0, 64, False),       # one tile
+    (1, 37, 64, True),       # two
+    (4, 0, 64, False), (16, 64, 64, False), (16, 1200, 64, True),
+    (8, 100, 128, False), (8, 900, 128, True),
+    (2, 100, 300, True),     # row blocks of one part and of more
+    (1, 0, 1000, True), (5, 800, 192, True), (1, 4000, 1, True),
+])
+def test_row_blocks_are_shared_out_where_it_pays(dev, batch, prior, lq, shared):
+    """Partials are written for enough keys per row and not otherwise: of many
+    short row blocks they cost more than the shorter chains save."""
+    call = _Call(dev, prior, lq, capacity=4096, batch=batch)
+    out = call.parts()
+    assert call.ws.any().item() == shared
+    _close(out, call.plain(), "parts")
     assert call.counters_are_zero()
