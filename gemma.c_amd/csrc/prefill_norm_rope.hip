@@ -135,9 +135,12 @@ __global__ __launch_bounds__((prep_waves<kHeads, kHasV>() * kWave)) void prefill
 }
 
 // ---- 1x512 causal self-attention ---------------------------------------
-// Up to this many rows the short form is faster (100 rows 21.3 against 23.4 us:
-// the long form fills its pipeline of three tiles first; 333 rows 34.6 / 34.1).
-constexpr int kD512ShortRows = 256;
+// Up to this many rows the short form is faster: the long form fills its
+// pipeline of three tiles first. Short / long, prep included, 1 / 2 / 4
+// sequences: 260 rows 28.6 / 30.5, 32.3 / 34.0, 39.3 / 45.0 us; 400 36.3 / 37.4,
+// 40.1 / 41.1, 59.8 / 62.5; 512 42.8 / 42.9, 45.9 / 45.5, 76.2 / 76.4; 700 52.4 /
+// 51.6, 58.5 / 57.5, 102.6 / 105.2.
+constexpr int kD512ShortRows = 512;
 constexpr int kD512 = 512;
 constexpr int kD512Rows = 4;          // query rows per workgroup, two waves each
 constexpr int kD512Waves = 2 * kD512Rows;

@@ -181,7 +181,8 @@ def test_launcher_argument_checks(dev):
 
 
 @pytest.mark.parametrize("batch,seq,weight", [
-    (1, 256, 1.0), (1, 257, 1.0), (2, 260, 8.0), (1, 287, 8.0), (1, 289, 1.0), (3, 320, 8.0), (1, 1030, 8.0)])
+    (1, 256, 1.0), (1, 257, 1.0), (2, 260, 8.0), (1, 287, 8.0), (1, 289, 1.0), (3, 320, 8.0), (1, 1030, 8.0),
+    (1, 512, 8.0), (1, 513, 1.0), (2, 516, 8.0), (1, 543, 8.0), (1, 545, 1.0), (3, 576, 8.0)])
 def test_global_long_and_short_forms(dev, batch, seq, weight):
     """Both 1 x 512 kernels around the length that separates them, at the
     edges of row groups and key tiles, against fp64 attention over the GPU's
