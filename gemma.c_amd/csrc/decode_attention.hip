@@ -614,19 +614,20 @@ __global__ __launch_bounds__(Sh::kMaxW * kWave) void decode_split_kernel(DecodeP
   // before the workgroup counts its arrival, so the last arriver's coherent
   // loads see every split. Whole-L2 write-back/invalidate is never needed.
   __shared__ int32_t s_last;
+  const int32_t arriving = min(live_splits, p.num_splits);  // the plan may cover fewer keys
   wait_stores_complete();
   __syncthreads();
   if (threadIdx.x == 0) {
     int32_t *counter = p.counters + (int64_t)b * c.num_heads + head;
     const int32_t arrived =
         __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool last = arrived == live_splits - 1;
+    const bool last = arrived == arriving - 1;
     if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s_last = last ? 1 : 0;
   }
   __syncthreads();
   if (s_last == 0 || key_lane != 0) return;
-  combine_row_group<GW, D, LPR, RPL>(p, b, head * G + hg * GW, live_splits, r, cpack);
+  combine_row_group<GW, D, LPR, RPL>(p, b, head * G + hg * GW, arriving, r, cpack);
 }
 
 // Log-sum-exp combine of the live splits of one (batch, query head) row

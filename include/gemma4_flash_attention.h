@@ -33,8 +33,8 @@ extern "C" {
 //                  (only gemma4_flash_attention_decode_split_paged_bf16
 //                  leaves partials to combine). Unused when num_splits == 1
 //                  (the single split writes d_out directly; may then be null).
-// The splits cover split_size * num_splits live keys from the first on; more
-// are not attended to. Supported geometries: (num_heads, head_dim) = (8, 256)
+// The splits cover split_size * num_splits live keys, from the first on (of a
+// full ring: from its first slot); more are not attended to. Supported geometries: (num_heads, head_dim) = (8, 256)
 // and (1, 512); 16 query heads.
 hipError_t gemma4_flash_attention_decode_paged_bf16(
     gemma4_bf16 *d_out, float *d_partial_m, float *d_partial_l,

@@ -517,3 +517,27 @@ def test_empty_sequence_with_split_counters(dev, heads, dim, split):
     assert np.array_equal(from_dev_bf16(cv).reshape(exp_v.shape), exp_v)
     assert_close(from_dev_bf16(out).reshape(exp.shape), exp, "empty sequence")
     assert not counters.any().item()
+
+
+@pytest.mark.parametrize("heads,dim,split,splits", [(8, 256, 32, 3), (1, 512, 64, 2), (1, 512, 96, 2)])
+def test_split_counters_with_a_plan_of_fewer_keys(dev, heads, dim, split, splits):
+    """A plan covers split * splits keys of a longer sequence, and its counters
+    count the splits that the launch has: rows written, counters back at zero."""
+    import torch
+    rng = np.random.default_rng(dim + split)
+    held = [300, 40, 230]
+    cfg = cache_config(1, 3, 16, 20, heads, dim, 0)
+    pt = fill_page_table(cfg, held)
+    ck, cv = (randn_bf16(rng, (3 * 20 * 16, heads, dim)) for _ in range(2))
+    q, k, v = (randn_bf16(rng, (3, h, dim)) for h in (16, heads, heads))
+    exp = oracle.decode_attention(q, ck, cv, pt, [min(n, split * splits) for n in held], cfg, 0, 0.05)
+    counters = torch.zeros(3 * heads, dtype=torch.int32, device=dev)
+    out = to_dev(np.full_like(q, 0x7FC0), dev)
+    pm, pl, pa = (torch.full((3 * 16 * splits * d,), float("nan"), device=dev) for d in (1, 1, dim))
+    gk.check(gk.flash_attention_append_decode_paged_bf16(
+        out, pm, pl, pa, to_dev(q, dev), to_dev(ck, dev), to_dev(cv, dev), to_dev(pt, dev),
+        to_dev(np.int32(held), dev), to_dev(np.int32([-1] * 3), dev), to_dev(k, dev), to_dev(v, dev),
+        gk.make_config(*cfg), 0, 0.05, split, splits, 3, split_counters=counters))
+    torch.cuda.synchronize()
+    assert_close(from_dev_bf16(out).reshape(exp.shape), exp, "covered keys")
+    assert not counters.any().item()
