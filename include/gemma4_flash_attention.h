@@ -34,8 +34,8 @@ extern "C" {
 //                  leaves partials to combine). Unused when num_splits == 1
 //                  (the single split writes d_out directly; may then be null).
 // The splits cover split_size * num_splits live keys, from the first on (of a
-// full ring: from its first slot); more are not attended to. Supported geometries: (num_heads, head_dim) = (8, 256)
-// and (1, 512); 16 query heads.
+// full ring: from its first slot); more are not attended to. Supported
+// geometries: (num_heads, head_dim) = (8, 256) and (1, 512); 16 query heads.
 hipError_t gemma4_flash_attention_decode_paged_bf16(
     gemma4_bf16 *d_out, float *d_partial_m, float *d_partial_l,
     float *d_partial_acc, const gemma4_bf16 *d_q, const gemma4_bf16 *d_cache_k,
