@@ -134,6 +134,12 @@ __global__ __launch_bounds__(kWaves *kWave, 1) void decode_split_d512_kernel(Dec
   const int h = lane & 15;  // key of the K operand, head of the others
   const int g = lane >> 4;
   const Gemma4KvCacheConfig &c = p.c;
+  // The arguments come cold from memory: all are asked for here, in one round
+  // trip. Left to the compiler, the later ones are read behind the cut below
+  // (24 sequences of 1-1500 keys 17.57 us, 17.31 so; one of 100 9.32, 9.26).
+  asm volatile("" ::"s"(p.out), "s"(p.q), "s"(p.cache_k), "s"(p.page_table), "s"(p.counters),
+               "s"(p.new_k), "s"(p.q_norm_weight), "s"(p.sin), "s"(c.page_size), "s"(p.q_scale),
+               "s"(p.gate), "s"(p.balanced));
   int32_t split = blockIdx.y, b = blockIdx.z;
   int32_t split_size = p.split_size;
   const bool balanced = kWaves == 2 && p.balanced != 0;
